@@ -390,6 +390,8 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_bf16_kernel(GemmArgs g) {
     }
 }
 
+#include "gemm_wide.hpp"
+
 // ---------------------------------------------------------------------------
 // Row statistics, embedding, RoPE + cache append.
 // ---------------------------------------------------------------------------
@@ -1310,6 +1312,27 @@ uint32_t gemm_gateup_split_rows(uint32_t N) {
 
 size_t gemm_split_elems(uint32_t M, uint32_t K) { return static_cast<size_t>(2) * M * gemm_kp(K); }
 
+// The 256 x 256 tile runs where its rounds over the CUs cost less than those
+// of the 128 x 256 tile. A round of it takes 1.63 times as long for twice the
+// work (64 K steps, gate/up at 2048 rows of 2048 x 8192: 2 rounds 217 us
+// against 4 rounds 264 us), so it loses only where its last round is emptier.
+// K splits keep the smaller tile: they exist to fill one round.
+static bool gemm_uses_wide(uint32_t M, uint32_t cols, uint32_t splits) {
+    const uint32_t cus = gemm_cus();
+    const uint32_t wide = ((cols + kWN - 1) / kWN) * ((M + kWM - 1) / kWM);
+    const uint32_t tile = ((cols + kBN - 1) / kBN) * ((M + kBM - 1) / kBM);
+    return splits == 1 && 5 * ((wide + cus - 1) / cus) <= 3 * ((tile + cus - 1) / cus);
+}
+
+template <int MODE>
+static hipError_t launch_gemm_wide(const GemmArgs& g, uint32_t cols, hipStream_t s) {
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_wide_kernel<MODE>),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, kWideLds);
+    if (attr != hipSuccess) return attr;
+    const dim3 grid(((cols + kWN - 1) / kWN) * ((g.M + kWM - 1) / kWM));
+    return vlaunch(gemm_wide_kernel<MODE>, grid, dim3(kGemmThreads), kWideLds, s, g);
+}
+
 hipError_t launch_gemm_bf16(int mode, const GemmArgs& g, hipStream_t s) {
     if (g.M == 0 || g.N == 0) return hipSuccess;
     if (!g.a_hl || g.K % 8 != 0 || (g.norm_w && !g.row_scale)) return hipErrorInvalidValue;
@@ -1351,6 +1374,11 @@ hipError_t launch_gemm_bf16(int mode, const GemmArgs& g, hipStream_t s) {
         hipError_t e = vlaunch(gemm_bf16_kernel<kGemmGateUp>, grid, dim3(kGemmThreads), kGemmLds, s, g);
         if (e != hipSuccess) return e;
         return vlaunch(gemm_swiglu_kernel, dim3((gemm_kp(g.N) + 255) / 256, g.M), dim3(256), 0, s, g);
+    }
+    if (gemm_uses_wide(g.M, cols, splits)) {
+        if (mode == kGemmPlain) return launch_gemm_wide<kGemmPlain>(g, cols, s);
+        if (mode == kGemmResid) return launch_gemm_wide<kGemmResid>(g, cols, s);
+        return launch_gemm_wide<kGemmGateUp>(g, cols, s);
     }
     const dim3 grid(gx * gy, 1, splits);  // tiles in the XCD-aware order of the kernel
     switch (mode) {
