@@ -331,12 +331,12 @@ int vvli_gpu_test_sampler_trace(const float* logits, uint32_t n, const vvli_gpu_
  * hipStream_t or NULL for the null stream. Asynchronous: returns after the
  * launch. M <= 3 (and M = 4 when W has few row tiles) runs the
  * GEMV kernel, one launch for all rows of X (one per row when they do not fit
- * its LDS); otherwise 4 <= M <= 64 one skinny MFMA kernel (W
- * read once, X split into two bf16 halves in registers so the products keep
- * about 16 bits of each f32 activation; few row tiles split K across blocks
- * and the last block of a tile sums the partials in a fixed order); M > 64 one
- * MFMA GEMM through planes of the split X. Results are deterministic except on
- * the GEMM path, whose split-K partial sums are added with atomics (the last
+ * its LDS); otherwise 4 <= M <= 128 one kernel that reads W once and splits X
+ * into two bf16 halves in registers, so that the products keep about 16 bits
+ * of each f32 activation (up to 64 rows one of two by shape; K splits are
+ * summed in a fixed order); larger M, and M > 64 on very tall W, one MFMA GEMM
+ * through planes of the split X. Results are deterministic except on that
+ * GEMM path, whose split-K partial sums are added with atomics (the last
  * bits may vary run to run). Scratch (K-split partials and counters, or the
  * GEMM's planes: about 4*M*K bytes) is kept per stream, allocated
  * stream-ordered, grown when needed and kept until the process ends (calls on
@@ -349,7 +349,7 @@ int vvli_gpu_linear(const uint16_t* dW, const float* dX, const uint16_t* dBias, 
  * capture, serving loops and harnesses that forbid hipMalloc). Same
  * arguments, kernels and results as vvli_gpu_linear. Where that call keeps a
  * stream-ordered scratch (M > 64: the activation planes, 4*M*ceil32(K)
- * bytes; 4 <= M <= 64 with few row tiles: K-split partials), this one uses a
+ * bytes; 4 <= M <= 128 with few row tiles: K-split partials), this one uses a
  * static device array of VVLI_LINEAR_NOALLOC_SCRATCH_BYTES (plus 64 KiB of
  * counters) on each GPU it runs on, held until the process ends; a call
  * needing more returns VVLI_INVALID_CONFIG before any launch.

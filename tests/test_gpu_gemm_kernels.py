@@ -45,6 +45,60 @@ def test_wide_tile(M, N, K, bias):
     check_linear(M, N, K, bias)
 
 
+# The few-row GEMM: each row tile (16, 32, 64, 128 rows) with ragged rows and
+# columns, K chunks with a tail, K splits and their sum, several items a block,
+# f32 rows at an address that the copies cannot take.
+@pytest.mark.parametrize("M,N,K,bias", [(7, 2049, 8192, True), (16, 20000, 2056, False), (17, 2100, 4104, True),
+                                        (31, 1000, 2056, True), (48, 777, 2040, False), (64, 300, 1000, True),
+                                        (65, 200, 40, False), (100, 8200, 520, True), (128, 130, 72, True),
+                                        (128, 2048, 8, False)])
+def test_few_rows(M, N, K, bias):
+    check_linear(M, N, K, bias)
+
+
+def test_few_rows_unaligned_and_repeated():
+    import torch
+
+    M, N, K = 33, 2048, 2048
+    w = (torch.randn(N, K, device="cuda") * 0.02).bfloat16()
+    pool = torch.randn(M * K + 1, device="cuda")
+    x = pool[1:].view(M, K)  # 4-byte aligned only
+    y, y2 = torch.empty(M, N, device="cuda"), torch.empty(M, N, device="cuda")
+    s = torch.cuda.current_stream().cuda_stream
+    R.linear(w.data_ptr(), x.data_ptr(), y.data_ptr(), M, N, K, None, s)
+    ref = x.double() @ w.double().t()
+    size = x.double().abs() @ w.double().abs().t()
+    assert float(((y.double() - ref).abs() / size).max()) <= 2.0**-16 + K * 2.0**-24
+    x = x.clone()
+    R.linear(w.data_ptr(), x.data_ptr(), y.data_ptr(), M, N, K, None, s)
+    R.linear(w.data_ptr(), x.data_ptr(), y2.data_ptr(), M, N, K, None, s)
+    torch.cuda.synchronize()
+    assert torch.equal(y, y2)  # the splits are added in a fixed order
+
+
+def test_few_rows_under_capture():
+    """A call that needed no scratch before its first use can still be captured
+    on a fresh stream, and replays give the eager result."""
+    import torch
+
+    M, N, K = 16, 2048, 2048
+    w = (torch.randn(N, K, device="cuda") * 0.02).bfloat16()
+    x = torch.randn(M, K, device="cuda")
+    y, e = torch.empty(M, N, device="cuda"), torch.empty(M, N, device="cuda")
+    R.linear(w.data_ptr(), x.data_ptr(), e.data_ptr(), M, N, K, None, torch.cuda.current_stream().cuda_stream)
+    st = torch.cuda.Stream()
+    st.wait_stream(torch.cuda.current_stream())
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=st):
+        R.linear(w.data_ptr(), x.data_ptr(), y.data_ptr(), M, N, K, None, torch.cuda.current_stream().cuda_stream)
+    for _ in range(3):
+        y.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert float((y - e).norm() / e.norm()) <= 1e-5  # sum orders of the same 16-bit products
+        x += 0  # eager work between the replays
+
+
 def rel_err(got, ref):
     return float(np.max(np.abs(got.astype(np.float64) - ref)) / np.max(np.abs(ref)))
 
@@ -79,3 +133,13 @@ def test_wide_tile_prefill():
                            num_attention_heads=72, num_key_value_heads=8, max_position_embeddings=4096,
                            rope_theta=1e6, rms_norm_eps=1e-6, tie_word_embeddings=True, architecture="qwen2",
                            qkv_bias=True), [2000])
+
+
+def test_few_row_prefill():
+    """Prompt parts on each row tile of the few-row GEMM and just past it,
+    behind cached rows: q|k|v with bias, gate/up, o and down with K splits and
+    K tails (width 448, 1000)."""
+    check_prefill(C.Config(vocab_size=300, hidden_size=448, intermediate_size=1000, num_hidden_layers=2,
+                           num_attention_heads=7, num_key_value_heads=1, max_position_embeddings=4096, rope_theta=1e6,
+                           rms_norm_eps=1e-6, tie_word_embeddings=True, architecture="qwen2", qkv_bias=True),
+                  [1, 16, 17, 32, 33, 64, 65, 100, 128, 129])

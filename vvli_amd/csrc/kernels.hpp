@@ -332,10 +332,16 @@ struct GemmArgs {
     // order (deterministic).
     float* part = nullptr;
 };
-// K splits a launch of launch_gemm_bf16 will use (1: no split), and the
+// K splits a launch of launch_gemm_bf16 will use (1: no split; the few-row
+// kernel splits only launches that are given `part`), and the
 // capacity of the partial sums buffer any launch needs (elements).
 uint32_t gemm_splits(int mode, const GemmArgs& g);
 size_t gemm_part_elems();
+// The few-row kernel (M <= kSlabMaxRows): the splits it uses for a Plain launch
+// that is given `part`, and the pass that adds them up: out[i] = sum of part[z * n + i].
+constexpr uint32_t kSlabMaxRows = 128;
+uint32_t gemm_slab_part_splits(uint32_t M, uint32_t N, uint32_t K);
+hipError_t launch_slab_reduce(const float* part, float* out, size_t n, uint32_t splits, hipStream_t s);
 __host__ __device__ inline uint32_t gemm_kp(uint32_t K) { return (K + 31) / 32 * 32; }
 size_t gemm_split_elems(uint32_t M, uint32_t K);
 // Most rows for which a GateUp GEMM of N outputs may split K (gu_acc of

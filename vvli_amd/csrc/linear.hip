@@ -22,7 +22,8 @@ namespace {
 // Rows from which one MFMA kernel replaces the GEMV kernel (linear_gemv.hpp,
 // up to 4 rows of x in one launch: 4 only where the skinny kernel would split
 // K across blocks, linear_uses_gemv); up to kSkinnyMaxRows the skinny kernel
-// below, beyond it the prefill GEMM.
+// below or the few-row GEMM (gemm_slab.hpp, up to kSlabMaxRows; linear_uses_slab),
+// beyond it the prefill GEMM.
 constexpr uint32_t kLinearGemmMinRows = 4;
 constexpr uint32_t kSkinnyMaxRows = 64;
 
@@ -377,7 +378,43 @@ bool linear_uses_gemv(uint32_t M, uint32_t N, uint32_t K) {
     return M == 4 && skinny_tiles(N) < 256 && (size_t)M * K * sizeof(float) <= kGemvMaxLds;
 }
 
-size_t linear_payload_bytes(uint32_t M, uint32_t N, uint32_t K) {
+// Which kernel runs M >= 4 rows (after the GEMV rule above). The few-row GEMM
+// of gemm_slab.hpp stages X in LDS once per 64 rows of W where the skinny
+// kernel fetches it from L2 for every 16 to 64, but splits K across blocks with
+// a second launch that adds the splits; its copies need 16-byte aligned
+// pointers. Up to 64 rows the cheaper of the two by these estimates (us, fitted
+// to both kernels over ten shapes and M = 5 .. 64, within 20 %): a block of the
+// skinny kernel moves about 40 KB per us; a chunk of the few-row GEMM takes
+// kChunkUs. Measured, skinny / few-row: 2048 x 8192 M = 16 22.2 / 11.4, M = 64
+// 44.7 / 16.0; 128256 x 2048 M = 16 132.7 / 96; 2048 x 2048 M = 8 6.4 / 7.7,
+// M = 33 12.8 / 9.5; 1152 x 896 M = 33 7.0 / 8.0. From 65 to 128 rows against
+// the split pass and the 128 x 256 tiles: the few-row GEMM while its items are
+// one round (2048 x 2048 M = 96 21.8 / 13.7; 8192 x 2048 M = 128 34.7 / 25.5),
+// the tiles beyond (18944 x 3584 M = 128 61 / 102).
+bool slab_beats_skinny(uint32_t M, uint32_t N, uint32_t K) {
+    const float rows = static_cast<float>(M), k = static_cast<float>(K);
+    const uint32_t ks0 = skinny_splits(N, K), blocks = skinny_tiles(N) * ks0;
+    const float skinny = 2.8f + (ks0 > 1 ? 5.f : 0.f) +
+                         static_cast<float>((blocks + 255) / 256) * (k / ks0) * (4.f * rows + 32.f * skinny_nt(N)) / 40e3f;
+    constexpr float kChunkUs[] = {0.5f, 0.65f, 0.95f, 0.95f};  // 16, 32, 64 rows
+    const uint32_t ks = gemm_slab_part_splits(M, N, K), tiles = (N + 63) / 64, chunks = ((K + 127) / 128 + ks - 1) / ks;
+    const float slab = 4.4f + (ks > 1 ? 2.6f : 0.f) +
+                       static_cast<float>((tiles * ks + 255) / 256 * chunks) * kChunkUs[(M - 1) / 16];
+    return slab < skinny;
+}
+
+bool linear_uses_slab(const uint16_t* dW, const float* dX, uint32_t M, uint32_t N, uint32_t K) {
+    if (M < kLinearGemmMinRows || M > kSlabMaxRows || linear_uses_gemv(M, N, K) ||
+        (reinterpret_cast<uintptr_t>(dW) | reinterpret_cast<uintptr_t>(dX)) % 16 != 0)
+        return false;
+    return M <= kSkinnyMaxRows ? slab_beats_skinny(M, N, K) : (N + 63) / 64 * gemm_slab_part_splits(M, N, K) <= 256;
+}
+
+size_t linear_payload_bytes(bool slab, uint32_t M, uint32_t N, uint32_t K) {
+    if (slab) {
+        const uint32_t ks = gemm_slab_part_splits(M, N, K);
+        return ks > 1 ? (size_t)ks * M * N * sizeof(float) : 0;
+    }
     if (M > kSkinnyMaxRows) return gemm_split_elems(M, K) * sizeof(uint16_t);
     if (linear_uses_gemv(M, N, K)) return 0;
     if (M >= kLinearGemmMinRows) {
@@ -389,8 +426,19 @@ size_t linear_payload_bytes(uint32_t M, uint32_t N, uint32_t K) {
 
 // Enqueue the op on s. scratch: kCounterBytes + linear_payload_bytes of
 // device memory laid out as above, or null when the payload is 0.
-int linear_enqueue(const uint16_t* dW, const float* dX, const uint16_t* dBias, float* dY, uint32_t M, uint32_t N,
-                   uint32_t K, hipStream_t s, char* scratch_mem) {
+int linear_enqueue(bool slab, const uint16_t* dW, const float* dX, const uint16_t* dBias, float* dY, uint32_t M,
+                   uint32_t N, uint32_t K, hipStream_t s, char* scratch_mem) {
+    if (slab) {
+        const uint32_t ks = gemm_slab_part_splits(M, N, K);
+        GemmArgs g;
+        g.a = dX, g.lda = K, g.w[0] = dW, g.bias[0] = dBias;
+        g.seg_end[0] = g.seg_end[1] = g.seg_end[2] = N;
+        g.out = dY, g.ldo = N, g.M = M, g.N = N, g.K = K;
+        if (ks > 1) g.part = reinterpret_cast<float*>(scratch_mem + kCounterBytes);
+        HIP_TRY(launch_gemm_bf16(kGemmPlain, g, s));
+        if (ks > 1) HIP_TRY(launch_slab_reduce(g.part, dY, (size_t)M * N, ks, s));
+        return VVLI_OK;
+    }
     if (M >= kLinearGemmMinRows && M <= kSkinnyMaxRows && !linear_uses_gemv(M, N, K)) {
         float* ws = scratch_mem ? reinterpret_cast<float*>(scratch_mem + kCounterBytes) : nullptr;
         uint32_t* cnt = reinterpret_cast<uint32_t*>(scratch_mem);
@@ -450,9 +498,10 @@ int vvli_gpu_linear(const uint16_t* dW, const float* dX, const uint16_t* dBias, 
     int rc = check_linear_args(dW, dX, dY, M, N, K, "vvli_gpu_linear");
     if (rc) return rc;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const size_t payload = linear_payload_bytes(M, N, K);
-    if (payload == 0) return linear_enqueue(dW, dX, dBias, dY, M, N, K, s, nullptr);
-    const size_t need = kCounterBytes + payload;
+    bool slab = linear_uses_slab(dW, dX, M, N, K);
+    size_t payload = linear_payload_bytes(slab, M, N, K);
+    if (payload == 0) return linear_enqueue(slab, dW, dX, dBias, dY, M, N, K, s, nullptr);
+    size_t need = kCounterBytes + payload;
     // The scratch is kept per stream and grows stream-ordered (its counters
     // cleared once per allocation); the lock covers the enqueue, so calls on
     // one stream use it in turn.
@@ -471,6 +520,18 @@ int vvli_gpu_linear(const uint16_t* dW, const float* dX, const uint16_t* dBias, 
         cache.push_back(StreamScratch{s, nullptr, 0});
         sc = &cache.back();
     }
+    if (slab && sc->bytes < need) {
+        // Under stream capture nothing may be allocated for a call that the
+        // other kernels serve without scratch: they take it.
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+            (void)hipGetLastError();
+            slab = false;
+            payload = linear_payload_bytes(slab, M, N, K);
+            if (payload == 0) return linear_enqueue(slab, dW, dX, dBias, dY, M, N, K, s, nullptr);
+            need = kCounterBytes + payload;
+        }
+    }
     if (sc->bytes < need) {
         if (sc->p) HIP_TRY(hipFreeAsync(sc->p, s));
         sc->p = nullptr, sc->bytes = 0;
@@ -478,21 +539,24 @@ int vvli_gpu_linear(const uint16_t* dW, const float* dX, const uint16_t* dBias, 
         HIP_TRY(hipMemsetAsync(sc->p, 0, kCounterBytes, s));
         sc->bytes = need;
     }
-    return linear_enqueue(dW, dX, dBias, dY, M, N, K, s, static_cast<char*>(sc->p));
+    return linear_enqueue(slab, dW, dX, dBias, dY, M, N, K, s, static_cast<char*>(sc->p));
 }
 
 int vvli_gpu_linear_noalloc(const uint16_t* dW, const float* dX, const uint16_t* dBias, float* dY, uint32_t M,
                             uint32_t N, uint32_t K, void* stream) {
     int rc = check_linear_args(dW, dX, dY, M, N, K, "vvli_gpu_linear_noalloc");
     if (rc) return rc;
-    const size_t payload = linear_payload_bytes(M, N, K);
-    if (payload > kNoAllocScratchBytes)
+    const bool slab = linear_uses_slab(dW, dX, M, N, K);
+    const size_t payload = linear_payload_bytes(slab, M, N, K);
+    // (The bound that callers know is that of the split planes, M > 64.)
+    const size_t bound = std::max(payload, linear_payload_bytes(false, M, N, K));
+    if (bound > kNoAllocScratchBytes)
         return set_error(VVLI_INVALID_CONFIG,
                          "vvli_gpu_linear_noalloc: M=%u N=%u K=%u needs %zu bytes of scratch, more than its %zu", M, N,
-                         K, payload, kNoAllocScratchBytes);
+                         K, bound, kNoAllocScratchBytes);
     char* mem = nullptr;
     if (payload && (rc = scratch_on_device(&mem))) return rc;
-    return linear_enqueue(dW, dX, dBias, dY, M, N, K, static_cast<hipStream_t>(stream), mem);
+    return linear_enqueue(slab, dW, dX, dBias, dY, M, N, K, static_cast<hipStream_t>(stream), mem);
 }
 
 }  // extern "C"

@@ -887,8 +887,9 @@ int enqueue_prefill_batched(vvli_gpu_model* m, uint32_t start, uint32_t n, uint3
     // atomic adds they replace -- measured at 128 rows, where down splits 32
     // ways: 3.11 ms with atomics, 3.30 ms with partial sums.)
     auto use_part = [&](int mode, GemmArgs& g) {
-        const uint32_t sp = m->pf_part ? gemm_splits(mode, g) : 1u;
-        g.part = (sp > 1 && sp <= 8) ? m->pf_part : nullptr;
+        g.part = m->pf_part;
+        const uint32_t sp = g.part ? gemm_splits(mode, g) : 1u;
+        if (sp < 2 || sp > 8) g.part = nullptr;
         return g.part ? sp : 0u;
     };
     for (uint32_t c0 = 0; c0 < n; c0 += m->pf_rows) {

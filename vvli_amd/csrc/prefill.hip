@@ -390,6 +390,7 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_bf16_kernel(GemmArgs g) {
     }
 }
 
+#include "gemm_slab.hpp"
 #include "gemm_wide.hpp"
 
 // ---------------------------------------------------------------------------
@@ -1287,9 +1288,88 @@ uint32_t gemm_k_splits(int mode, const GemmArgs& g, uint32_t tiles) {
     return splits;
 }
 
-uint32_t gemm_splits(int mode, const GemmArgs& g) {
+// The 256 x 256 tile runs where its rounds over the CUs cost less than those
+// of the 128 x 256 tile. A round of it takes 1.63 times as long for twice the
+// work (64 K steps, gate/up at 2048 rows of 2048 x 8192: 2 rounds 217 us
+// against 4 rounds 264 us), so it loses only where its last round is emptier.
+// K splits keep the smaller tile: they exist to fill one round.
+static bool gemm_uses_wide(uint32_t M, uint32_t cols, uint32_t splits) {
+    const uint32_t cus = gemm_cus();
+    const uint32_t wide = ((cols + kWN - 1) / kWN) * ((M + kWM - 1) / kWM);
+    const uint32_t tile = ((cols + kBN - 1) / kBN) * ((M + kBM - 1) / kBM);
+    return splits == 1 && 5 * ((wide + cus - 1) / cus) <= 3 * ((tile + cus - 1) / cus);
+}
+
+template <int MODE>
+static hipError_t launch_gemm_wide(const GemmArgs& g, uint32_t cols, hipStream_t s) {
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_wide_kernel<MODE>),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, kWideLds);
+    if (attr != hipSuccess) return attr;
+    const dim3 grid(((cols + kWN - 1) / kWN) * ((g.M + kWM - 1) / kWM));
+    return vlaunch(gemm_wide_kernel<MODE>, grid, dim3(kGemmThreads), kWideLds, s, g);
+}
+
+// Which kernel a launch runs and its K splits.
+enum class GemmKernel { Tile, Wide, Slab };
+struct GemmPlan {
+    GemmKernel kernel;
+    uint32_t splits;
+};
+
+// Splits of the few-row kernel: enough items for a block per CU, the fewest
+// splits with the same longest K range, at most kMaxPartSplits.
+static uint32_t slab_splits(uint32_t tiles, uint32_t K, uint32_t M) {
+    const uint32_t kc = M > 64 ? 64 : 128, nch = (K + kc - 1) / kc;
+    const uint32_t most = std::max(1u, std::min({gemm_cus() / tiles, kMaxPartSplits, nch}));
+    const uint32_t per = (nch + most - 1) / most;
+    return (nch + per - 1) / per;
+}
+
+static GemmPlan gemm_plan(int mode, const GemmArgs& g) {
     const uint32_t cols = mode == kGemmGateUp ? 2 * g.N : g.N;
-    return gemm_k_splits(mode, g, ((cols + kBN - 1) / kBN) * ((g.M + kBM - 1) / kBM));
+    // Few rows: the slab kernel. Up to 64 rows always (one layer of the 1B
+    // shape at 45 rows: gate/up 36 -> 20 us with its zeroing and SwiGLU passes,
+    // o and down 17 -> 9.5, q|k|v 15 -> 9.5); from 65 to 128 while its items
+    // are one round (8192 x 2048 at 128 rows 25.5 us against 34.7 on the
+    // tiles, 18944 x 3584 102 against 61).
+    if (g.M <= kSlabMaxRows && (mode != kGemmPlain || g.ldo == g.N || !g.part)) {
+        const uint32_t tiles = (cols + kSlabN - 1) / kSlabN;
+        const uint32_t splits = mode != kGemmGateUp && g.part ? slab_splits(tiles, g.K, g.M) : 1u;
+        if (g.M <= 64 || tiles * splits <= gemm_cus()) return {GemmKernel::Slab, splits};
+    }
+    const uint32_t gx = (cols + kBN - 1) / kBN, gy = (g.M + kBM - 1) / kBM;
+    const uint32_t splits = gemm_k_splits(mode, g, gx * gy);
+    if (gemm_uses_wide(g.M, cols, splits)) return {GemmKernel::Wide, 1};
+    return {GemmKernel::Tile, splits};
+}
+
+uint32_t gemm_splits(int mode, const GemmArgs& g) { return gemm_plan(mode, g).splits; }
+
+uint32_t gemm_slab_part_splits(uint32_t M, uint32_t N, uint32_t K) {
+    return M <= kSlabMaxRows ? slab_splits((N + kSlabN - 1) / kSlabN, K, M) : 1;
+}
+
+template <int MODE, int MT, int KC, int ST, int WM, int WN, bool F32A>
+static hipError_t launch_slab_t(const GemmArgs& g, uint32_t splits, hipStream_t s) {
+    using S = SlabShape<MT, KC, ST, WM, WN>;
+    static const hipError_t attr =
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_slab_kernel<MODE, MT, KC, ST, WM, WN, F32A>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, S::Lds);
+    if (attr != hipSuccess) return attr;
+    const uint32_t cols = MODE == kGemmGateUp ? 2 * g.N : g.N, tiles = (cols + kSlabN - 1) / kSlabN;
+    const uint32_t items = tiles * splits;
+    // Blocks take items in whole rounds: the fewest that give the same rounds.
+    const uint32_t cus = gemm_cus(), rounds = (items + cus - 1) / cus;
+    return vlaunch(gemm_slab_kernel<MODE, MT, KC, ST, WM, WN, F32A>, dim3((items + rounds - 1) / rounds),
+                   dim3(kSlabThreads), S::Lds, s, g, tiles, splits);
+}
+
+template <int MODE, bool F32A>
+static hipError_t launch_slab(const GemmArgs& g, uint32_t splits, hipStream_t s) {
+    if (g.M <= 16) return launch_slab_t<MODE, 1, 128, 6, 1, 2, F32A>(g, splits, s);
+    if (g.M <= 32) return launch_slab_t<MODE, 2, 128, 4, 2, 1, F32A>(g, splits, s);
+    if (g.M <= 64) return launch_slab_t<MODE, 4, 128, 3, 4, 1, F32A>(g, splits, s);
+    return launch_slab_t<MODE, 8, 64, 3, 4, 1, F32A>(g, splits, s);
 }
 
 size_t gemm_part_elems() { return static_cast<size_t>(gemm_cus()) * kBM * kBN; }
@@ -1312,38 +1392,27 @@ uint32_t gemm_gateup_split_rows(uint32_t N) {
 
 size_t gemm_split_elems(uint32_t M, uint32_t K) { return static_cast<size_t>(2) * M * gemm_kp(K); }
 
-// The 256 x 256 tile runs where its rounds over the CUs cost less than those
-// of the 128 x 256 tile. A round of it takes 1.63 times as long for twice the
-// work (64 K steps, gate/up at 2048 rows of 2048 x 8192: 2 rounds 217 us
-// against 4 rounds 264 us), so it loses only where its last round is emptier.
-// K splits keep the smaller tile: they exist to fill one round.
-static bool gemm_uses_wide(uint32_t M, uint32_t cols, uint32_t splits) {
-    const uint32_t cus = gemm_cus();
-    const uint32_t wide = ((cols + kWN - 1) / kWN) * ((M + kWM - 1) / kWM);
-    const uint32_t tile = ((cols + kBN - 1) / kBN) * ((M + kBM - 1) / kBM);
-    return splits == 1 && 5 * ((wide + cus - 1) / cus) <= 3 * ((tile + cus - 1) / cus);
-}
-
-template <int MODE>
-static hipError_t launch_gemm_wide(const GemmArgs& g, uint32_t cols, hipStream_t s) {
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_wide_kernel<MODE>),
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize, kWideLds);
-    if (attr != hipSuccess) return attr;
-    const dim3 grid(((cols + kWN - 1) / kWN) * ((g.M + kWM - 1) / kWM));
-    return vlaunch(gemm_wide_kernel<MODE>, grid, dim3(kGemmThreads), kWideLds, s, g);
-}
-
 hipError_t launch_gemm_bf16(int mode, const GemmArgs& g, hipStream_t s) {
     if (g.M == 0 || g.N == 0) return hipSuccess;
-    if (!g.a_hl || g.K % 8 != 0 || (g.norm_w && !g.row_scale)) return hipErrorInvalidValue;
+    const GemmPlan plan = gemm_plan(mode, g);
+    // The few-row kernel splits f32 rows itself.
+    const bool f32a = plan.kernel == GemmKernel::Slab && mode == kGemmPlain && !g.a_ready && !g.norm_w && !g.a_rows &&
+                      g.a && g.lda % 4 == 0 && reinterpret_cast<uintptr_t>(g.a) % 16 == 0;
+    if ((!g.a_hl && !f32a) || g.K % 8 != 0 || (g.norm_w && !g.row_scale)) return hipErrorInvalidValue;
     if ((g.out_hl && mode != kGemmGateUp) || (!g.out_hl && !g.out) ||
         (g.a_plane && g.a_plane < static_cast<size_t>(g.M) * gemm_kp(g.K)) ||
         (g.out_hl && g.out_plane < static_cast<size_t>(g.M) * gemm_kp(g.N)))
         return hipErrorInvalidValue;
-    if (!g.a_ready) {
+    if (!g.a_ready && !f32a) {
         const size_t n = static_cast<size_t>(g.M) * (gemm_kp(g.K) / 8);
         hipError_t e = vlaunch(gemm_split_kernel, dim3(static_cast<uint32_t>((n + 255) / 256)), dim3(256), 0, s, g);
         if (e != hipSuccess) return e;
+    }
+    if (plan.kernel == GemmKernel::Slab) {
+        if (plan.splits > 1 && static_cast<size_t>(plan.splits) * g.M * g.N > gemm_part_elems()) return hipErrorInvalidValue;
+        if (mode == kGemmGateUp) return launch_slab<kGemmGateUp, false>(g, plan.splits, s);
+        if (mode == kGemmResid) return launch_slab<kGemmResid, false>(g, plan.splits, s);
+        return f32a ? launch_slab<kGemmPlain, true>(g, plan.splits, s) : launch_slab<kGemmPlain, false>(g, plan.splits, s);
     }
     static const hipError_t attr = [] {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_bf16_kernel<kGemmPlain>),
@@ -1359,7 +1428,7 @@ hipError_t launch_gemm_bf16(int mode, const GemmArgs& g, hipStream_t s) {
     if (attr != hipSuccess) return attr;
     const uint32_t cols = mode == kGemmGateUp ? 2 * g.N : g.N;
     const uint32_t gx = (cols + kBN - 1) / kBN, gy = (g.M + kBM - 1) / kBM;
-    const uint32_t splits = gemm_k_splits(mode, g, gx * gy);
+    const uint32_t splits = plan.splits;
     if (splits > 1 && g.part && static_cast<size_t>(splits) * g.M * g.N > gemm_part_elems())
         return hipErrorInvalidValue;  // (splits * tiles <= CUs keeps every launch within it)
     if (splits > 1 && mode != kGemmResid && !(mode == kGemmPlain && g.part)) {
@@ -1375,7 +1444,7 @@ hipError_t launch_gemm_bf16(int mode, const GemmArgs& g, hipStream_t s) {
         if (e != hipSuccess) return e;
         return vlaunch(gemm_swiglu_kernel, dim3((gemm_kp(g.N) + 255) / 256, g.M), dim3(256), 0, s, g);
     }
-    if (gemm_uses_wide(g.M, cols, splits)) {
+    if (plan.kernel == GemmKernel::Wide) {
         if (mode == kGemmPlain) return launch_gemm_wide<kGemmPlain>(g, cols, s);
         if (mode == kGemmResid) return launch_gemm_wide<kGemmResid>(g, cols, s);
         return launch_gemm_wide<kGemmGateUp>(g, cols, s);
@@ -1387,6 +1456,12 @@ hipError_t launch_gemm_bf16(int mode, const GemmArgs& g, hipStream_t s) {
         case kGemmGateUp: return vlaunch(gemm_bf16_kernel<kGemmGateUp>, grid, dim3(kGemmThreads), kGemmLds, s, g);
         default: return hipErrorInvalidValue;
     }
+}
+
+hipError_t launch_slab_reduce(const float* part, float* out, size_t n, uint32_t splits, hipStream_t s) {
+    if (splits > kMaxPartSplits || n > gemm_part_elems()) return hipErrorInvalidValue;
+    return vlaunch(slab_reduce_kernel, dim3(static_cast<uint32_t>((n + 255) / 256)), dim3(256), 0, s, part, out,
+                   static_cast<uint32_t>(n), splits);
 }
 
 uint32_t grouped_gemm_tile_rows() { return kBM; }
