@@ -270,8 +270,9 @@ int vvli_gpu_profile_step(vvli_gpu_model* model, uint32_t token, uint32_t pos, f
  * checking both against the same reference. */
 int vvli_gpu_set_decode_path(vvli_gpu_model* model, uint32_t path);
 /* How vvli_gpu_prefill (and generate with VVLI_GEN_BATCHED_PREFILL) runs the
- * prompt: 0 = auto (batched where supported), 1 = token loop, 2 = batched
- * (VVLI_INVALID_CONFIG if the model does not support it). */
+ * prompt: 0 = auto (batched where supported; f32 weights in f32 throughout),
+ * 1 = token loop, 2 = batched with bf16 weights (VVLI_INVALID_CONFIG if the
+ * model does not support it). */
 int vvli_gpu_set_prefill_path(vvli_gpu_model* model, uint32_t path);
 /* One persistent step with phase timestamps (100 MHz ticks): ticks_out holds
  * (n_blocks + 1) * stride values. With stride >= 16 * (5 * layers + 2), phase

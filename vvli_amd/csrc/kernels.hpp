@@ -356,6 +356,31 @@ uint32_t grouped_gemm_max_tiles(uint32_t M, uint32_t E);
 // no bias): each tile of g.tiles multiplies its rows by its expert's W.
 hipError_t launch_gemm_grouped(int mode, const GemmArgs& g, hipStream_t s);
 
+// ---------------------------------------------------------------------------
+// f32 weights (prefill_f32.hip): out = a . w^T with f32 MFMA products.
+// ---------------------------------------------------------------------------
+struct F32GemmArgs {
+    const float* a = nullptr;  // [M][lda]
+    uint32_t lda = 0;
+    const float* w[3] = {nullptr, nullptr, nullptr};  // [rows][K] segments (GateUp: w[0] = gate)
+    const float* bias[3] = {nullptr, nullptr, nullptr};
+    uint32_t seg_end[3] = {0, 0, 0};  // cumulative rows of the segments, seg_end[2] = N
+    const float* w_up = nullptr;      // GateUp: up rows
+    float* out = nullptr;
+    uint32_t ldo = 0;
+    uint32_t M = 0, N = 0, K = 0;     // K % 4 == 0, lda % 4 == 0
+    // Plain / Resid: when set and the launch splits K (gemm_f32_splits > 1),
+    // the splits' sums [split][M][N] for the consumer, as GemmArgs::part.
+    float* part = nullptr;
+};
+uint32_t gemm_f32_splits(int mode, const F32GemmArgs& g);
+hipError_t launch_gemm_f32(int mode, const F32GemmArgs& g, hipStream_t s);
+// y = rmsnorm(x) with weight w, after x += part sums (as launch_row_norm_split).
+hipError_t launch_row_norm_f32(float* x, uint32_t n, uint32_t rows, float eps, const float* w, const float* part,
+                               uint32_t splits, float* y, hipStream_t s);
+hipError_t launch_embed_rows_f32(const float* embed, const uint32_t* tokens, uint32_t rows, uint32_t n, float* x,
+                                 hipStream_t s);
+
 // part / splits: the K-split partial sums of the Resid GEMM that produced x
 // ([splits][rows][n]; nullptr or splits <= 1: x is complete), added into x first.
 hipError_t launch_row_rms(float* x, uint32_t n, uint32_t rows, float eps, float* scale, hipStream_t s,
@@ -420,6 +445,8 @@ struct PrefillAttnArgs {
 // cache rows (0 for an unsupported head_dim).
 size_t prefill_kv_pack_bytes(uint32_t keys, uint32_t kv_heads, uint32_t hd);
 hipError_t launch_prefill_attn(const PrefillAttnArgs& a, uint32_t hd, hipStream_t s);
+// The same in f32 throughout (prefill_f32.hip; head_dim 32, 64 or 128).
+hipError_t launch_attn_f32(const PrefillAttnArgs& a, uint32_t hd, hipStream_t s);
 // false (default): the MFMA flash-attention kernel; true: the f32 vector kernel.
 extern bool prefill_attn_vector;
 // Form of the MFMA flash-attention launch: -1 chosen by the prompt (default),

@@ -97,7 +97,7 @@ struct vvli_gpu_model {
     uint32_t* sample_nf = nullptr;              // finite counts of the vocab slices
     void* sample_full = nullptr;                // whole-vocabulary candidates (limits over 1024)
     hipGraphExec_t graph_sample = nullptr;    // token step ending in the sampler
-    // Batched prefill (bf16 only): chunk buffers, allocated on first use.
+    // Batched prefill: chunk buffers, allocated on first use.
     bool pf_ok = false;
     uint32_t prefill_path = 0;  // 0 auto, 1 token loop, 2 batched
     uint32_t pf_rows = 0;       // rows per chunk the buffers hold
@@ -105,8 +105,8 @@ struct vvli_gpu_model {
     float* pf_qkv = nullptr;    // [rows][H + 2 kv]
     float* pf_attn = nullptr;   // [rows][H]
     float* pf_scale = nullptr;  // [rows] RMS scales
-    float* pf_ahl = nullptr;    // GEMM activations split hi | lo (gemm_split_elems bf16)
-    float* pf_ahl2 = nullptr;   // split planes written by attention (o_proj's A) and SwiGLU (down's A)
+    float* pf_ahl = nullptr;    // GEMM activations split hi | lo (gemm_split_elems bf16); f32 weights: normed rows
+    float* pf_ahl2 = nullptr;   // split planes written by attention (o_proj's A) and SwiGLU (down's A); f32 weights: SwiGLU rows
     float* pf_gu = nullptr;     // gate/up split-K sums for short chunks ([pf_gu_rows][2I])
     float* pf_part = nullptr;   // K-split partial sums of q|k|v, o_proj and down (gemm_part_elems)
     uint32_t pf_gu_rows = 0;
@@ -743,7 +743,8 @@ int read_outputs(vvli_gpu_model* m, float* logits_out, uint32_t* argmax_out) {
 // ---------------------------------------------------------------------------
 // Batched prefill: every prompt row of a chunk through each layer at once
 // (prefill.hip). Same KV rows and last logits as the token loop, within the
-// f32 tolerance; bf16 weights and head_dim 32 / 64 / 128.
+// f32 tolerance; head_dim 32 / 64 / 128. What follows is for bf16 weights;
+// enqueue_prefill_layers_f32 runs the layers of f32 ones.
 // ---------------------------------------------------------------------------
 constexpr uint32_t kPrefillChunk = 2048;  // rows per pass; bounds the chunk buffers
 
@@ -752,8 +753,20 @@ bool prefill_supported(const vvli_gpu_config& c) {
     return c.weight_kind == VVLI_WEIGHT_BF16 && (hd == 32 || hd == 64 || hd == 128);
 }
 
-bool use_batched_prefill(const vvli_gpu_model* m) {
-    return m->prefill_path != 1 && prefill_supported(m->cfg);
+// f32 weights take the batched prefill of prefill_f32.hip (path 2 asks for the
+// bf16 one; 1 is the token loop).
+bool prefill_f32_supported(const vvli_gpu_config& c) {
+    const uint32_t hd = head_dim(c);
+    return c.weight_kind == VVLI_WEIGHT_F32 && (hd == 32 || hd == 64 || hd == 128);
+}
+
+int ensure_prefill_buffers(vvli_gpu_model* m);
+
+bool use_batched_prefill(vvli_gpu_model* m) {
+    if (m->prefill_path == 1) return false;
+    if (prefill_supported(m->cfg)) return true;
+    // (the token loop needs no chunk buffers: it serves where they do not fit)
+    return prefill_f32_supported(m->cfg) && ensure_prefill_buffers(m) == VVLI_OK;
 }
 
 int ensure_prefill_buffers(vvli_gpu_model* m) {
@@ -775,8 +788,9 @@ int ensure_prefill_buffers(vvli_gpu_model* m) {
                              "prefill buffers (%zu rows): %s", rows, hipGetErrorString(e));
         }
     }
-    const size_t kvp = prefill_kv_pack_bytes(static_cast<uint32_t>(m->max_seq), c.kv_heads, head_dim(c));
-    hipError_t e = hipMalloc(&m->pf_kvp, kvp);
+    const bool f32 = c.weight_kind == VVLI_WEIGHT_F32;  // (its attention reads the cache rows themselves)
+    const size_t kvp = f32 ? 0 : prefill_kv_pack_bytes(static_cast<uint32_t>(m->max_seq), c.kv_heads, head_dim(c));
+    hipError_t e = f32 ? hipSuccess : hipMalloc(&m->pf_kvp, kvp);
     if (e != hipSuccess) {
         for (float** b : bufs) {
             (void)hipFree(*b);
@@ -793,7 +807,7 @@ int ensure_prefill_buffers(vvli_gpu_model* m) {
         m->pf_part = nullptr;  // split GEMMs then add their partial sums atomically
         (void)hipGetLastError();
     }
-    if (m->moe) return VVLI_OK;
+    if (m->moe || f32) return VVLI_OK;
     const uint32_t gu_rows = std::min<uint32_t>(m->pf_rows, gemm_gateup_split_rows(c.inter));
     if (gu_rows > 0 && hipMalloc(reinterpret_cast<void**>(&m->pf_gu), static_cast<size_t>(gu_rows) * 2 * I *
                                                                           sizeof(float)) == hipSuccess)
@@ -866,6 +880,56 @@ int enqueue_prefill_moe_ffn(vvli_gpu_model* m, uint32_t l, uint32_t P, hipStream
     return VVLI_OK;
 }
 
+// The layers of a chunk with f32 weights: rows pos0 .. pos0 + P - 1 of pf_x
+// (embedded) through every layer, left complete in pf_x.
+int enqueue_prefill_layers_f32(vvli_gpu_model* m, uint32_t pos0, uint32_t P, hipStream_t s) {
+    const vvli_gpu_config& c = m->cfg;
+    const uint32_t H = c.hidden, kv = kv_dim(c), I = c.inter, hd = head_dim(c), ldqkv = H + 2 * kv;
+    float* const normed = m->pf_ahl;  // [P][H]
+    float* const ff = m->pf_ahl2;     // [P][I]
+    auto w = [&](size_t off) { return static_cast<const float*>(wslice(m, off)); };
+    auto product = [&](int mode, F32GemmArgs& g, const float* a, uint32_t lda, float* out, uint32_t ldo, uint32_t N,
+                       uint32_t K) {
+        g.a = a, g.lda = lda, g.out = out, g.ldo = ldo, g.M = P, g.N = N, g.K = K, g.part = m->pf_part;
+        if (!g.seg_end[2]) g.seg_end[0] = g.seg_end[1] = g.seg_end[2] = N;
+        return launch_gemm_f32(mode, g, s);
+    };
+    uint32_t pend = 0;  // K splits of the product whose sums x still lacks
+    for (uint32_t l = 0; l < c.layers; ++l) {
+        const LayerSlices& L = m->layout.layers[l];
+        float* kc = m->kcache + static_cast<size_t>(l) * m->max_seq * kv;
+        float* vc = m->vcache + static_cast<size_t>(l) * m->max_seq * kv;
+        LAUNCH(launch_row_norm_f32(m->pf_x, H, P, c.rms_eps, w(L.input_norm), m->pf_part, pend, normed, s));
+        F32GemmArgs gq;
+        gq.w[0] = w(L.q), gq.w[1] = w(L.k), gq.w[2] = w(L.v);
+        gq.bias[0] = w(L.q_bias), gq.bias[1] = w(L.k_bias), gq.bias[2] = w(L.v_bias);
+        gq.seg_end[0] = H, gq.seg_end[1] = H + kv, gq.seg_end[2] = ldqkv;
+        LAUNCH(product(kGemmPlain, gq, normed, H, m->pf_qkv, ldqkv, ldqkv, H));
+        PrefillRopeArgs ra{m->pf_qkv, ldqkv, P, pos0, c.heads, c.kv_heads, hd, kv, c.rope_layout, m->rope_cs, kc, vc};
+        const uint32_t q_splits = gemm_f32_splits(kGemmPlain, gq);
+        if (q_splits > 1) ra.part = m->pf_part, ra.splits = q_splits;
+        LAUNCH(launch_prefill_rope_kv(ra, s));
+        PrefillAttnArgs aa{m->pf_qkv, ldqkv, kc, vc, m->pf_attn, H, P, pos0, c.heads, c.kv_heads, kv,
+                           1.0f / sqrtf(static_cast<float>(hd))};
+        LAUNCH(launch_attn_f32(aa, hd, s));
+        F32GemmArgs go;
+        go.w[0] = w(L.o);
+        LAUNCH(product(kGemmResid, go, m->pf_attn, H, m->pf_x, H, H, H));
+        pend = gemm_f32_splits(kGemmResid, go);
+        LAUNCH(launch_row_norm_f32(m->pf_x, H, P, c.rms_eps, w(L.post_norm), m->pf_part, pend, normed, s));
+        F32GemmArgs gu;
+        gu.w[0] = w(L.gate), gu.w_up = w(L.up);
+        LAUNCH(product(kGemmGateUp, gu, normed, H, ff, I, I, H));
+        F32GemmArgs gd;
+        gd.w[0] = w(L.down);
+        LAUNCH(product(kGemmResid, gd, ff, I, m->pf_x, H, H, I));
+        pend = gemm_f32_splits(kGemmResid, gd);
+    }
+    if (pend > 1)  // the last down projection's partial sums (the scale computed with them is unused)
+        LAUNCH(launch_row_rms(m->pf_x, H, P, c.rms_eps, m->pf_scale, s, m->pf_part, pend));
+    return VVLI_OK;
+}
+
 // Prompt tokens are already in m->prompt[start .. start + n). Leaves the KV
 // rows of those positions, the last row's logits and argmax, and the step
 // state as the token loop leaves it (next position start + n, next token the
@@ -896,8 +960,15 @@ int enqueue_prefill_batched(vvli_gpu_model* m, uint32_t start, uint32_t n, uint3
         const uint32_t P = std::min(m->pf_rows, n - c0);
         const uint32_t pos0 = start + c0;
         uint32_t pend = 0;
-        LAUNCH(launch_prefill_embed(embed, m->prompt + pos0, P, H, m->pf_x, s));
-        for (uint32_t l = 0; l < c.layers; ++l) {
+        const bool f32 = c.weight_kind == VVLI_WEIGHT_F32;
+        if (f32) {
+            LAUNCH(launch_embed_rows_f32(static_cast<const float*>(wslice(m, m->layout.embed)), m->prompt + pos0, P, H,
+                                         m->pf_x, s));
+            if ((rc = enqueue_prefill_layers_f32(m, pos0, P, s))) return rc;
+        } else {
+            LAUNCH(launch_prefill_embed(embed, m->prompt + pos0, P, H, m->pf_x, s));
+        }
+        for (uint32_t l = 0; !f32 && l < c.layers; ++l) {
             AttnSlices L;
             if (m->moe) {
                 const MoeLayerSlices& M = m->moe_layout.layers[l];

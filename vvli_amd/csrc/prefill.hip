@@ -428,22 +428,6 @@ __global__ __launch_bounds__(kRowThreads) void row_rms_kernel(float* __restrict_
     if (lane == 0) scale[wave] = 1.0f / sqrtf(acc / static_cast<float>(n) + eps);
 }
 
-// Up to 8 K-split partial sums of one float4 (stride elements apart), loaded
-// together, added onto v in split order.
-constexpr uint32_t kMaxPartSplits = 8;
-__device__ __forceinline__ float4 add_parts(float4 v, const float* __restrict__ p, size_t stride, uint32_t splits) {
-    float4 q[kMaxPartSplits];
-#pragma unroll
-    for (uint32_t z = 0; z < kMaxPartSplits; ++z)
-        q[z] = z < splits ? *reinterpret_cast<const float4*>(p + z * stride) : make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-    for (uint32_t z = 0; z < kMaxPartSplits; ++z)
-        if (z < splits)
-            v.x = __fadd_rn(v.x, q[z].x), v.y = __fadd_rn(v.y, q[z].y), v.z = __fadd_rn(v.z, q[z].z),
-            v.w = __fadd_rn(v.w, q[z].w);
-    return v;
-}
-
 // As row_rms_kernel with partial sums (at most kMaxPartSplits), a block per
 // row: x_r = x_r + p_0 + p_1 + ... (split order), written back, then the
 // row's scale.
