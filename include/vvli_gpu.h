@@ -337,9 +337,10 @@ int vvli_gpu_test_sampler_trace(const float* logits, uint32_t n, const vvli_gpu_
  * of each f32 activation (up to 64 rows one of two by shape; K splits are
  * summed in a fixed order); larger M, and M > 64 on very tall W, one MFMA GEMM
  * through planes of the split X. Results are deterministic except on that
- * GEMM path, whose split-K partial sums are added with atomics (the last
- * bits may vary run to run). Scratch (K-split partials and counters, or the
- * GEMM's planes: about 4*M*K bytes) is kept per stream, allocated
+ * GEMM path where K is split more than eight ways, or the partial sums find
+ * no scratch under capture: they are then added with atomics (the last bits
+ * may vary run to run). Scratch (K-split partials and counters, or the
+ * GEMM's planes, about 4*M*K bytes, and its K-split partials, at most 32 MiB) is kept per stream, allocated
  * stream-ordered, grown when needed and kept until the process ends (calls on
  * one stream use it in turn). */
 int vvli_gpu_linear(const uint16_t* dW, const float* dX, const uint16_t* dBias, float* dY, uint32_t M, uint32_t N,
@@ -352,8 +353,9 @@ int vvli_gpu_linear(const uint16_t* dW, const float* dX, const uint16_t* dBias, 
  * stream-ordered scratch (M > 64: the activation planes, 4*M*ceil32(K)
  * bytes; 4 <= M <= 128 with few row tiles: K-split partials), this one uses a
  * static device array of VVLI_LINEAR_NOALLOC_SCRATCH_BYTES (plus 64 KiB of
- * counters) on each GPU it runs on, held until the process ends; a call
- * needing more returns VVLI_INVALID_CONFIG before any launch.
+ * counters and 32 MiB for the K-split partials of M > 64) on each GPU it runs
+ * on, held until the process ends; a call needing more returns
+ * VVLI_INVALID_CONFIG before any launch.
  * The array of the current device is used (stream must belong to it). Every
  * call on one GPU shares that array and nothing in it needs clearing, but
  * calls that overlap on one GPU (other streams, other threads) race on it:

@@ -143,3 +143,47 @@ def test_few_row_prefill():
                            num_attention_heads=7, num_key_value_heads=1, max_position_embeddings=4096, rope_theta=1e6,
                            rms_norm_eps=1e-6, tie_word_embeddings=True, architecture="qwen2", qkv_bias=True),
                   [1, 16, 17, 32, 33, 64, 65, 100, 128, 129])
+
+
+# The 128 x 128 tile: fewer than its three stages of 64 and an odd and even
+# number of them, K tails of 8 to 56, ragged rows and columns, one block, a
+# full round, K splits that are summed by a pass of their own.
+@pytest.mark.parametrize("M,N,K,bias", [(129, 100, 8, True), (250, 300, 72, False), (200, 5000, 200, True),
+                                        (512, 8192, 136, False), (512, 8190, 504, True), (300, 1000, 2056, True),
+                                        (131, 1001, 4024, False), (700, 513, 8192, True)])
+def test_square_tile(M, N, K, bias):
+    check_linear(M, N, K, bias)
+
+
+def test_square_tile_prefill():
+    """q|k|v with bias, gate/up, o and down with K splits and K tails (width
+    448, 1000) behind cached rows, at the row counts around its tiles."""
+    check_prefill(C.Config(vocab_size=300, hidden_size=448, intermediate_size=1000, num_hidden_layers=2,
+                           num_attention_heads=7, num_key_value_heads=1, max_position_embeddings=4096, rope_theta=1e6,
+                           rms_norm_eps=1e-6, tie_word_embeddings=True, architecture="qwen2", qkv_bias=True),
+                  [140, 256, 257, 520])
+
+
+def test_square_tile_under_capture():
+    """A K-split call captured with scratch for its split planes alone (a
+    smaller call came before it on that stream) takes no more of it."""
+    import torch
+
+    K = 2048
+    w = (torch.randn(2048, K, device="cuda") * 0.02).bfloat16()
+    x = torch.randn(512, K, device="cuda")
+    y, e = torch.empty(512, 2048, device="cuda"), torch.empty(512, 2048, device="cuda")
+    st = torch.cuda.Stream()
+    R.linear(w.data_ptr(), x.data_ptr(), e.data_ptr(), 512, 2048, K, None, torch.cuda.current_stream().cuda_stream)
+    st.wait_stream(torch.cuda.current_stream())
+    R.linear(w.data_ptr(), x.data_ptr(), y.data_ptr(), 512, 16, K, None, st.cuda_stream)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=st):
+        R.linear(w.data_ptr(), x.data_ptr(), y.data_ptr(), 512, 2048, K, None, torch.cuda.current_stream().cuda_stream)
+    for _ in range(3):
+        y.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert float((y - e).norm() / e.norm()) <= 1e-5  # sum orders of the same 16-bit products
+        x += 0  # eager work between the replays

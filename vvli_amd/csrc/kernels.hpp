@@ -336,9 +336,12 @@ struct GemmArgs {
 // kernel splits only launches that are given `part`), and the
 // capacity of the partial sums buffer any launch needs (elements).
 uint32_t gemm_splits(int mode, const GemmArgs& g);
+// gemm_splits of a dense Plain launch that is given `part`.
+uint32_t gemm_plain_part_splits(uint32_t M, uint32_t N, uint32_t K);
 size_t gemm_part_elems();
 // The few-row kernel (M <= kSlabMaxRows): the splits it uses for a Plain launch
-// that is given `part`, and the pass that adds them up: out[i] = sum of part[z * n + i].
+// that is given `part`. launch_slab_reduce adds up any Plain launch's splits:
+// out[i] = sum of part[z * n + i].
 constexpr uint32_t kSlabMaxRows = 128;
 uint32_t gemm_slab_part_splits(uint32_t M, uint32_t N, uint32_t K);
 hipError_t launch_slab_reduce(const float* part, float* out, size_t n, uint32_t splits, hipStream_t s);

@@ -305,7 +305,10 @@ hipError_t launch_skinny(const uint16_t* dW, const float* dX, const uint16_t* dB
 // device (scratch_on_device).
 constexpr size_t kCounterBytes = 64 * 1024;
 constexpr size_t kNoAllocScratchBytes = static_cast<size_t>(VVLI_LINEAR_NOALLOC_SCRATCH_BYTES);
-static __device__ __align__(256) uint16_t scratch[(kCounterBytes + kNoAllocScratchBytes) / sizeof(uint16_t)];
+// Room behind it for the partial sums of a K split (gemm_part_elems on 256
+// CUs): both entry points then run the same kernels on the same splits.
+constexpr size_t kNoAllocPartBytes = static_cast<size_t>(32) << 20;
+static __device__ __align__(256) uint16_t scratch[(kCounterBytes + kNoAllocScratchBytes + kNoAllocPartBytes) / sizeof(uint16_t)];
 
 constexpr int kMaxDevices = 64;
 
@@ -410,12 +413,21 @@ bool linear_uses_slab(const uint16_t* dW, const float* dX, uint32_t M, uint32_t 
     return M <= kSkinnyMaxRows ? slab_beats_skinny(M, N, K) : (N + 63) / 64 * gemm_slab_part_splits(M, N, K) <= 256;
 }
 
+// M > 64: the split planes, and behind them the partial sums of a K split
+// (0: the launch does not split K, or more ways than the summing pass takes).
+size_t linear_plane_bytes(uint32_t M, uint32_t K) { return gemm_split_elems(M, K) * sizeof(uint16_t); }
+size_t linear_part_bytes(uint32_t M, uint32_t N, uint32_t K) {
+    if (M <= kSkinnyMaxRows) return 0;
+    const uint32_t ks = gemm_plain_part_splits(M, N, K);
+    return ks > 1 && ks <= 8 ? (size_t)ks * M * N * sizeof(float) : 0;
+}
+
 size_t linear_payload_bytes(bool slab, uint32_t M, uint32_t N, uint32_t K) {
     if (slab) {
         const uint32_t ks = gemm_slab_part_splits(M, N, K);
         return ks > 1 ? (size_t)ks * M * N * sizeof(float) : 0;
     }
-    if (M > kSkinnyMaxRows) return gemm_split_elems(M, K) * sizeof(uint16_t);
+    if (M > kSkinnyMaxRows) return linear_plane_bytes(M, K);
     if (linear_uses_gemv(M, N, K)) return 0;
     if (M >= kLinearGemmMinRows) {
         const uint32_t ks = skinny_splits(N, K);
@@ -425,8 +437,9 @@ size_t linear_payload_bytes(bool slab, uint32_t M, uint32_t N, uint32_t K) {
 }
 
 // Enqueue the op on s. scratch: kCounterBytes + linear_payload_bytes of
-// device memory laid out as above, or null when the payload is 0.
-int linear_enqueue(bool slab, const uint16_t* dW, const float* dX, const uint16_t* dBias, float* dY, uint32_t M,
+// device memory laid out as above (and linear_part_bytes behind them with
+// `parts`: else the splits add atomically), or null when the payload is 0.
+int linear_enqueue(bool slab, bool parts, const uint16_t* dW, const float* dX, const uint16_t* dBias, float* dY, uint32_t M,
                    uint32_t N, uint32_t K, hipStream_t s, char* scratch_mem) {
     if (slab) {
         const uint32_t ks = gemm_slab_part_splits(M, N, K);
@@ -453,7 +466,9 @@ int linear_enqueue(bool slab, const uint16_t* dW, const float* dX, const uint16_
         g.seg_end[0] = g.seg_end[1] = g.seg_end[2] = N;
         g.out = dY, g.ldo = N, g.M = M, g.N = N, g.K = K;
         g.a_hl = reinterpret_cast<uint16_t*>(scratch_mem + kCounterBytes);
+        if (parts) g.part = reinterpret_cast<float*>(scratch_mem + kCounterBytes + linear_plane_bytes(M, K));
         HIP_TRY(launch_gemm_bf16(kGemmPlain, g, s));
+        if (parts) HIP_TRY(launch_slab_reduce(g.part, dY, (size_t)M * N, gemm_splits(kGemmPlain, g), s));
         return VVLI_OK;
     }
     // M <= 4: one GEMV launch for all rows when their x fits LDS, else one per row.
@@ -500,8 +515,10 @@ int vvli_gpu_linear(const uint16_t* dW, const float* dX, const uint16_t* dBias, 
     hipStream_t s = static_cast<hipStream_t>(stream);
     bool slab = linear_uses_slab(dW, dX, M, N, K);
     size_t payload = linear_payload_bytes(slab, M, N, K);
-    if (payload == 0) return linear_enqueue(slab, dW, dX, dBias, dY, M, N, K, s, nullptr);
-    size_t need = kCounterBytes + payload;
+    if (payload == 0) return linear_enqueue(slab, false, dW, dX, dBias, dY, M, N, K, s, nullptr);
+    const size_t part_bytes = slab ? 0 : linear_part_bytes(M, N, K);
+    bool parts = part_bytes > 0;
+    size_t need = kCounterBytes + payload + part_bytes;
     // The scratch is kept per stream and grows stream-ordered (its counters
     // cleared once per allocation); the lock covers the enqueue, so calls on
     // one stream use it in turn.
@@ -520,15 +537,15 @@ int vvli_gpu_linear(const uint16_t* dW, const float* dX, const uint16_t* dBias, 
         cache.push_back(StreamScratch{s, nullptr, 0});
         sc = &cache.back();
     }
-    if (slab && sc->bytes < need) {
+    if ((slab || parts) && sc->bytes < need) {
         // Under stream capture nothing may be allocated for a call that the
-        // other kernels serve without scratch: they take it.
+        // other kernels serve without scratch or with less: they take it.
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
             (void)hipGetLastError();
-            slab = false;
+            slab = parts = false;
             payload = linear_payload_bytes(slab, M, N, K);
-            if (payload == 0) return linear_enqueue(slab, dW, dX, dBias, dY, M, N, K, s, nullptr);
+            if (payload == 0) return linear_enqueue(slab, parts, dW, dX, dBias, dY, M, N, K, s, nullptr);
             need = kCounterBytes + payload;
         }
     }
@@ -539,7 +556,7 @@ int vvli_gpu_linear(const uint16_t* dW, const float* dX, const uint16_t* dBias, 
         HIP_TRY(hipMemsetAsync(sc->p, 0, kCounterBytes, s));
         sc->bytes = need;
     }
-    return linear_enqueue(slab, dW, dX, dBias, dY, M, N, K, s, static_cast<char*>(sc->p));
+    return linear_enqueue(slab, parts, dW, dX, dBias, dY, M, N, K, s, static_cast<char*>(sc->p));
 }
 
 int vvli_gpu_linear_noalloc(const uint16_t* dW, const float* dX, const uint16_t* dBias, float* dY, uint32_t M,
@@ -554,9 +571,11 @@ int vvli_gpu_linear_noalloc(const uint16_t* dW, const float* dX, const uint16_t*
         return set_error(VVLI_INVALID_CONFIG,
                          "vvli_gpu_linear_noalloc: M=%u N=%u K=%u needs %zu bytes of scratch, more than its %zu", M, N,
                          K, bound, kNoAllocScratchBytes);
+    const size_t part_bytes = slab ? 0 : linear_part_bytes(M, N, K);
+    const bool parts = part_bytes > 0 && part_bytes <= kNoAllocPartBytes;
     char* mem = nullptr;
     if (payload && (rc = scratch_on_device(&mem))) return rc;
-    return linear_enqueue(slab, dW, dX, dBias, dY, M, N, K, static_cast<hipStream_t>(stream), mem);
+    return linear_enqueue(slab, parts, dW, dX, dBias, dY, M, N, K, static_cast<hipStream_t>(stream), mem);
 }
 
 }  // extern "C"

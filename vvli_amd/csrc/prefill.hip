@@ -392,6 +392,7 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_bf16_kernel(GemmArgs g) {
 
 #include "gemm_slab.hpp"
 #include "gemm_wide.hpp"
+#include "gemm_square.hpp"
 
 // ---------------------------------------------------------------------------
 // Row statistics, embedding, RoPE + cache append.
@@ -1272,16 +1273,53 @@ uint32_t gemm_k_splits(int mode, const GemmArgs& g, uint32_t tiles) {
     return splits;
 }
 
-// The 256 x 256 tile runs where its rounds over the CUs cost less than those
-// of the 128 x 256 tile. A round of it takes 1.63 times as long for twice the
-// work (64 K steps, gate/up at 2048 rows of 2048 x 8192: 2 rounds 217 us
-// against 4 rounds 264 us), so it loses only where its last round is emptier.
-// K splits keep the smaller tile: they exist to fill one round.
-static bool gemm_uses_wide(uint32_t M, uint32_t cols, uint32_t splits) {
-    const uint32_t cus = gemm_cus();
-    const uint32_t wide = ((cols + kWN - 1) / kWN) * ((M + kWM - 1) / kWM);
-    const uint32_t tile = ((cols + kBN - 1) / kBN) * ((M + kBM - 1) / kBM);
-    return splits == 1 && 5 * ((wide + cus - 1) / cus) <= 3 * ((tile + cus - 1) / cus);
+size_t gemm_part_elems() { return static_cast<size_t>(gemm_cus()) * kBM * kBN; }
+
+// What a launch costs on each tile, in us: a round over the CUs takes 7 to 7.5
+// us and, per K step of 32, 0.90 on 128 x 256, 1.48 on 256 x 256, 0.47 on
+// 128 x 128; a K split adds its partial sums, written and read once by their
+// consumer (5 MB per us, and up to 3 us for a launch or its loads), or zeroing
+// and atomic adds (1.7 MB per us). Fitted to linear on each of the three (us, 128 x
+// 256 / 256 x 256 / 128 x 128): 2048 x 8192 x 2048 147 / 118 / 158, with K 512
+// 60 / 47 / 70; 2048 x 4096 x 2048 80 / 100 / 87; 512 x 8192 x 2048 55 / 97 /
+// 46; 512 x 18000 x 1000 83 / 63 / 78; 200 x 2048 x 8192 50 / 320 / 35;
+// 130 x 1000 x 4000 29 / 159 / 26.
+static float gemm_tile_us(int mode, const GemmArgs& g, uint32_t cols, uint32_t splits) {
+    const uint32_t cus = gemm_cus(), nk = (g.K + kBK - 1) / kBK;
+    const uint32_t tiles = ((cols + kBN - 1) / kBN) * ((g.M + kBM - 1) / kBM);
+    const float mb = 4e-6f * splits * g.M * cols;
+    float us = ((tiles * splits + cus - 1) / cus) * (7.5f + 0.9f * ((nk + splits - 1) / splits));
+    if (splits > 1) us += g.part && mode != kGemmGateUp ? 3.f + mb / 2.5f : 3.f + mb / 1.7f;
+    if (splits > 1 && mode == kGemmGateUp) us += 5.f;  // the SwiGLU pass
+    return us;
+}
+static float gemm_wide_us(const GemmArgs& g, uint32_t cols) {
+    const uint32_t cus = gemm_cus(), tiles = ((cols + kWN - 1) / kWN) * ((g.M + kWM - 1) / kWM);
+    return ((tiles + cus - 1) / cus) * (7.f + 1.48f * ((g.K + kBK - 1) / kBK));
+}
+// (splits: the best for the tile, at least four stages of K each)
+static float gemm_square_us(int mode, const GemmArgs& g, uint32_t cols, uint32_t& splits) {
+    const uint32_t cus = gemm_cus(), tiles = ((cols + kSqN - 1) / kSqN) * ((g.M + kSqM - 1) / kSqM);
+    const uint32_t nk = (g.K + kSqK - 1) / kSqK;
+    const uint32_t most = mode != kGemmGateUp && g.part ? std::max(1u, std::min(kMaxPartSplits, nk / 4)) : 1u;
+    float best = 0.f;
+    for (uint32_t want = 1; want <= most; ++want) {
+        const uint32_t per = (nk + want - 1) / want, sp = (nk + per - 1) / per;  // every split gets K steps
+        if (sp > 1 && static_cast<size_t>(sp) * g.M * g.N > gemm_part_elems()) break;
+        float us = ((tiles * sp + cus - 1) / cus) * (7.f + 0.94f * per);
+        if (sp > 1) us += (mode == kGemmResid ? 0.5f : 3.f) + 4e-6f * sp * g.M * g.N / 2.5f;
+        if (want == 1 || us < best) best = us, splits = sp;
+    }
+    return best;
+}
+
+template <int MODE>
+static hipError_t launch_gemm_square(const GemmArgs& g, uint32_t cols, uint32_t splits, hipStream_t s) {
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_square_kernel<MODE>),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, kSqLds);
+    if (attr != hipSuccess) return attr;
+    const dim3 grid(((cols + kSqN - 1) / kSqN) * ((g.M + kSqM - 1) / kSqM), 1, splits);
+    return vlaunch(gemm_square_kernel<MODE>, grid, dim3(kGemmThreads), kSqLds, s, g);
 }
 
 template <int MODE>
@@ -1294,7 +1332,7 @@ static hipError_t launch_gemm_wide(const GemmArgs& g, uint32_t cols, hipStream_t
 }
 
 // Which kernel a launch runs and its K splits.
-enum class GemmKernel { Tile, Wide, Slab };
+enum class GemmKernel { Tile, Wide, Slab, Square };
 struct GemmPlan {
     GemmKernel kernel;
     uint32_t splits;
@@ -1323,11 +1361,22 @@ static GemmPlan gemm_plan(int mode, const GemmArgs& g) {
     }
     const uint32_t gx = (cols + kBN - 1) / kBN, gy = (g.M + kBM - 1) / kBM;
     const uint32_t splits = gemm_k_splits(mode, g, gx * gy);
-    if (gemm_uses_wide(g.M, cols, splits)) return {GemmKernel::Wide, 1};
+    uint32_t sq_splits = 1;
+    const float tile = gemm_tile_us(mode, g, cols, splits), wide = gemm_wide_us(g, cols);
+    const float square = gemm_square_us(mode, g, cols, sq_splits);
+    if (square < tile && square < wide) return {GemmKernel::Square, sq_splits};
+    if (wide < tile) return {GemmKernel::Wide, 1};
     return {GemmKernel::Tile, splits};
 }
 
 uint32_t gemm_splits(int mode, const GemmArgs& g) { return gemm_plan(mode, g).splits; }
+
+uint32_t gemm_plain_part_splits(uint32_t M, uint32_t N, uint32_t K) {
+    static float there;  // only that `part` is given counts
+    GemmArgs g;
+    g.M = M, g.N = N, g.K = K, g.ldo = N, g.part = &there;
+    return gemm_plan(kGemmPlain, g).splits;
+}
 
 uint32_t gemm_slab_part_splits(uint32_t M, uint32_t N, uint32_t K) {
     return M <= kSlabMaxRows ? slab_splits((N + kSlabN - 1) / kSlabN, K, M) : 1;
@@ -1355,8 +1404,6 @@ static hipError_t launch_slab(const GemmArgs& g, uint32_t splits, hipStream_t s)
     if (g.M <= 64) return launch_slab_t<MODE, 4, 128, 3, 4, 1, F32A>(g, splits, s);
     return launch_slab_t<MODE, 8, 64, 3, 4, 1, F32A>(g, splits, s);
 }
-
-size_t gemm_part_elems() { return static_cast<size_t>(gemm_cus()) * kBM * kBN; }
 
 static uint32_t fa_tile_keys(uint32_t hd) { return hd == 128 ? FaShape<128>::TK : FaShape<64>::TK; }
 static_assert(FaShape<32>::Stage == 8 * 64 * 32 && FaShape<64>::Stage == 8 * 64 * 64 &&
@@ -1415,6 +1462,11 @@ hipError_t launch_gemm_bf16(int mode, const GemmArgs& g, hipStream_t s) {
     const uint32_t splits = plan.splits;
     if (splits > 1 && g.part && static_cast<size_t>(splits) * g.M * g.N > gemm_part_elems())
         return hipErrorInvalidValue;  // (splits * tiles <= CUs keeps every launch within it)
+    if (plan.kernel == GemmKernel::Square) {
+        if (mode == kGemmPlain) return launch_gemm_square<kGemmPlain>(g, cols, splits, s);
+        if (mode == kGemmResid) return launch_gemm_square<kGemmResid>(g, cols, splits, s);
+        return launch_gemm_square<kGemmGateUp>(g, cols, splits, s);
+    }
     if (splits > 1 && mode != kGemmResid && !(mode == kGemmPlain && g.part)) {
         const bool gu = mode == kGemmGateUp;
         const size_t n = static_cast<size_t>(g.M) * (gu ? 2 * g.N : g.ldo);
