@@ -72,7 +72,13 @@ __device__ __forceinline__ void slab_split(f32x4 a, f32x4 b, bf16x8& hi, bf16x8&
     }
 }
 
-template <int MODE, int MT, int KC, int ST, int WM, int WN, bool F32A>
+// Grouped launches (rows of a mixture's experts): an item is 64 rows of an
+// expert's W for one entry of the tile table, columns fastest, so that the
+// blocks stream one expert after another. The table moves to LDS at the start:
+// read from memory, an entry would wait behind the copies in flight.
+constexpr uint32_t kSlabTable = 512;  // entries of 8 bytes: first row; expert, rows
+
+template <int MODE, int MT, int KC, int ST, int WM, int WN, bool F32A, bool GROUPED>
 __global__ __launch_bounds__(kSlabThreads) void gemm_slab_kernel(GemmArgs g, uint32_t tiles, uint32_t splits) {
     using S = SlabShape<MT, KC, ST, WM, WN>;
     constexpr int WK = S::WK, MW = MT / WM, NW = 4 / WN;  // MFMA tiles of a wave: MW x NW
@@ -86,14 +92,38 @@ __global__ __launch_bounds__(kSlabThreads) void gemm_slab_kernel(GemmArgs g, uin
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wn = wave % WN, wm = wave / WN % WM, wk = wave / (WN * WM);
-    const uint32_t items = tiles * splits;
+    uint32_t items = tiles * splits;
+    const uint32_t table = gemm_lds_addr(gemm_smem) + S::Lds;
+    if (GROUPED) {
+        const uint32_t count = min(g.tiles[0].x, kSlabTable);
+        uint2* tab = reinterpret_cast<uint2*>(gemm_smem + S::Lds);
+        for (uint32_t t = tid; t < count; t += kSlabThreads) {
+            const uint4 td = g.tiles[1 + t];
+            tab[t] = make_uint2(td.y, td.x << 16 | (td.z - td.y));
+        }
+        items = tiles * static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(count));
+        __syncthreads();
+    }
+    // Item i of a grouped launch: first row, rows, expert.
+    struct Group {
+        uint32_t m0, rows, expert;
+    };
+    auto group = [&](uint32_t i) {
+        if (!GROUPED) return Group{0, g.M, 0};
+        vvli_u32x2 v;
+        asm volatile("ds_read_b64 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(v) : "v"(table + i / tiles * 8));
+        const uint32_t y = __builtin_amdgcn_readfirstlane(v.y);
+        return Group{static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(v.x)), y & 0xffffu, y >> 16};
+    };
     const uint32_t nch = (g.K + KC - 1) / KC, per = (nch + splits - 1) / splits;
     const uint32_t kp = gemm_kp(g.K);
     const size_t plane = g.a_plane ? g.a_plane : static_cast<size_t>(g.M) * kp;
 
-    // Copy sources. A: row and 16-byte chunk of each copy are fixed.
+    // Copy sources. A: the 16-byte chunk of each copy is fixed, the row too
+    // unless the launch is grouped.
     const char* srcA[PA];
     uint32_t kA[PA];
+    auto set_a = [&](uint32_t m0, uint32_t rows) {
 #pragma unroll
     for (int i = 0; i < PA; ++i) {
         constexpr int Rows = 64 / ALanes;  // rows per copy
@@ -101,7 +131,7 @@ __global__ __launch_bounds__(kSlabThreads) void gemm_slab_kernel(GemmArgs g, uin
         const uint32_t lr = q * Rows + lane / ALanes;  // row within the A stage (planes: hi rows, then lo rows)
         const uint32_t r = F32A ? lr : lr % (MT * 16);
         const uint32_t c = (lane % ALanes) ^ (r & (ALanes >= 16 ? 15u : 7u));
-        const uint32_t m = min(r, g.M - 1);  // rows past M repeat the last (never written)
+        const uint32_t m = m0 + min(r, rows - 1);  // rows past the end repeat the last (never written)
         if (F32A) {
             kA[i] = c * 4;
             srcA[i] = reinterpret_cast<const char*>(g.a + static_cast<size_t>(m) * g.lda + kA[i]);
@@ -111,17 +141,19 @@ __global__ __launch_bounds__(kSlabThreads) void gemm_slab_kernel(GemmArgs g, uin
                                                     kA[i]);
         }
     }
+    };
+    if (!GROUPED) set_a(0, g.M);
     const char* srcW[PW];
     uint32_t kW[PW];
     constexpr int WRows = 64 / WLanes;
     const uint32_t wrow0 = wave * PW * WRows + lane / WLanes;
-    auto set_w = [&](uint32_t n0) {
+    auto set_w = [&](uint32_t n0, size_t eoff) {
 #pragma unroll
         for (int i = 0; i < PW; ++i) {
             const uint32_t row = wrow0 + i * WRows;
             kW[i] = ((lane % WLanes) ^ (row & (WLanes >= 16 ? 15u : 7u))) * 8;
             bool valid;
-            srcW[i] = reinterpret_cast<const char*>(gemm_w_row<MODE>(g, n0, static_cast<int>(row), 0, valid) + kW[i]);
+            srcW[i] = reinterpret_cast<const char*>(gemm_w_row<MODE>(g, n0, static_cast<int>(row), eoff, valid) + kW[i]);
         }
     };
     // Issue side: the next chunk to copy.
@@ -130,7 +162,13 @@ __global__ __launch_bounds__(kSlabThreads) void gemm_slab_kernel(GemmArgs g, uin
         const uint32_t z = ii % splits;
         ib = z * per, il = min(per, nch - ib);
         iat = (ii / splits / 8) % il, ileft = il;
-        set_w(ii / splits * kSlabN);
+        if (GROUPED) {
+            const Group gr = group(ii);
+            set_a(gr.m0, gr.rows);
+            set_w(ii % tiles * kSlabN, static_cast<size_t>(gr.expert) * g.w_expert);
+            return;
+        }
+        set_w(ii / splits * kSlabN, 0);
     };
     auto issue = [&]() {
         if (ii >= items) return;  // uniform
@@ -242,7 +280,8 @@ __global__ __launch_bounds__(kSlabThreads) void gemm_slab_kernel(GemmArgs g, uin
         static_assert(Steps <= 2, "counted waits for at most two steps");
         if (++cc != cn) continue;
         // Item done: the WK partial sums in LDS, then the epilogue.
-        const uint32_t n0 = ci / splits * kSlabN, z = ci % splits;
+        const uint32_t n0 = (GROUPED ? ci % tiles : ci / splits) * kSlabN, z = GROUPED ? 0 : ci % splits;
+        const Group gr = group(ci);
         const uint32_t red = lds0 + ST * S::Stage + (wm * WN + wn) * (MW * NW * 1024) + lane * 16;
         constexpr uint32_t kRedK = WM * WN * MW * NW * 1024;  // bytes of one K group's sums
         if (wk > 0) {
@@ -273,8 +312,8 @@ __global__ __launch_bounds__(kSlabThreads) void gemm_slab_kernel(GemmArgs g, uin
             for (int i = 0; i < MW; ++i) {
 #pragma unroll
                 for (int jr = 0; jr < 4; ++jr) {
-                    const uint32_t row = (wm * MW + i) * 16 + 4 * fq + jr;
-                    if (row >= g.M) continue;
+                    const uint32_t lrow = (wm * MW + i) * 16 + 4 * fq + jr, row = gr.m0 + lrow;
+                    if (lrow >= gr.rows) continue;
                     if (MODE == kGemmGateUp) {
                         const uint32_t kpo = gemm_kp(g.N);
 #pragma unroll

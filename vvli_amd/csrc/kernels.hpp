@@ -322,7 +322,7 @@ struct GemmArgs {
     // tiles[1 + t] = {expert, first row, end row, 0} (rows of the A planes and
     // of the output); the expert's W is w[0] (and w_up) + expert * w_expert.
     const uint4* tiles = nullptr;
-    uint32_t max_tiles = 0;
+    uint32_t max_tiles = 0, tile_rows = 0;  // (grouped_gemm_max_tiles, grouped_gemm_tile_rows)
     size_t w_expert = 0;
     // Plain / Resid: when set and the launch splits K (gemm_splits > 1), each
     // split stores its partial sums to part[split][M][N] (f32, at most
@@ -351,9 +351,9 @@ size_t gemm_split_elems(uint32_t M, uint32_t K);
 // rows * 2N floats is then needed).
 uint32_t gemm_gateup_split_rows(uint32_t N);
 hipError_t launch_gemm_bf16(int mode, const GemmArgs& g, hipStream_t s);
-// Rows of one grouped GEMM tile; a table for M grouped rows over E experts
+// Rows of a grouped GEMM's tiles for M grouped rows over E experts; their table
 // holds at most grouped_gemm_max_tiles(M, E) tiles.
-uint32_t grouped_gemm_tile_rows();
+uint32_t grouped_gemm_tile_rows(uint32_t M, uint32_t E);
 uint32_t grouped_gemm_max_tiles(uint32_t M, uint32_t E);
 // Per-expert GEMMs over grouped rows (kGemmGateUp or kGemmPlain; no K split,
 // no bias): each tile of g.tiles multiplies its rows by its expert's W.

@@ -825,7 +825,8 @@ int ensure_moe_prefill_buffers(vvli_gpu_model* m) {
                      reinterpret_cast<void**>(&m->pf_grows), reinterpret_cast<void**>(&m->pf_ppos),
                      reinterpret_cast<void**>(&m->pf_tiles), reinterpret_cast<void**>(&m->pf_ehl),
                      reinterpret_cast<void**>(&m->pf_eact), reinterpret_cast<void**>(&m->pf_eout)};
-    const size_t tiles = 1 + grouped_gemm_max_tiles(static_cast<uint32_t>(n), c.num_experts);
+    // (the most tiles of any row count: shorter prompts use smaller tiles, up to 512 of them)
+    const size_t tiles = 1 + std::max<size_t>(grouped_gemm_max_tiles(static_cast<uint32_t>(n), c.num_experts), 512);
     const size_t bytes[] = {n * 4, n * 4, n * 4, n * 4, tiles * sizeof(uint4), gemm_split_elems(static_cast<uint32_t>(n), c.hidden) * 2,
                             gemm_split_elems(static_cast<uint32_t>(n), c.inter) * 2, n * c.hidden * sizeof(float)};
     for (int i = 0; i < 8; ++i) {
@@ -856,7 +857,7 @@ int enqueue_prefill_moe_ffn(vvli_gpu_model* m, uint32_t l, uint32_t P, hipStream
     ra.w = w16(L.router), ra.x = m->pf_x, ra.row_scale = m->pf_scale, ra.norm_w = w16(L.post_norm);
     ra.rows = P, ra.H = H, ra.E = E, ra.top_k = K, ra.idx = m->pf_eidx, ra.weight = m->pf_ew;
     LAUNCH(launch_moe_route_rows(ra, s));
-    LAUNCH(launch_moe_group(m->pf_eidx, P, K, E, grouped_gemm_tile_rows(), m->pf_grows, m->pf_ppos, m->pf_tiles, s));
+    LAUNCH(launch_moe_group(m->pf_eidx, P, K, E, grouped_gemm_tile_rows(n, E), m->pf_grows, m->pf_ppos, m->pf_tiles, s));
     // act = silu(norm(x_row) . Wg_e^T) * (norm(x_row) . Wu_e^T) per pair, as split planes
     GemmArgs gu;
     gu.a = m->pf_x, gu.lda = H, gu.a_rows = m->pf_grows, gu.row_scale = m->pf_scale, gu.norm_w = w16(L.post_norm);
@@ -866,7 +867,7 @@ int enqueue_prefill_moe_ffn(vvli_gpu_model* m, uint32_t l, uint32_t P, hipStream
     gu.M = n, gu.N = I, gu.K = H;
     gu.a_hl = m->pf_ehl;
     gu.out_hl = m->pf_eact, gu.out_plane = static_cast<size_t>(n) * gemm_kp(I);
-    gu.tiles = m->pf_tiles, gu.max_tiles = grouped_gemm_max_tiles(n, E);
+    gu.tiles = m->pf_tiles, gu.max_tiles = grouped_gemm_max_tiles(n, E), gu.tile_rows = grouped_gemm_tile_rows(n, E);
     LAUNCH(launch_gemm_grouped(kGemmGateUp, gu, s));
     // out_pair = act . Wd_e^T
     GemmArgs gd;
@@ -874,7 +875,7 @@ int enqueue_prefill_moe_ffn(vvli_gpu_model* m, uint32_t l, uint32_t P, hipStream
     gd.seg_end[0] = gd.seg_end[1] = gd.seg_end[2] = H;
     gd.out = m->pf_eout, gd.ldo = H, gd.M = n, gd.N = H, gd.K = I;
     gd.a_hl = m->pf_eact, gd.a_ready = true, gd.a_plane = static_cast<size_t>(n) * gemm_kp(I);
-    gd.tiles = m->pf_tiles, gd.max_tiles = gu.max_tiles;
+    gd.tiles = m->pf_tiles, gd.max_tiles = gu.max_tiles, gd.tile_rows = gu.tile_rows;
     LAUNCH(launch_gemm_grouped(kGemmPlain, gd, s));
     LAUNCH(launch_moe_combine(m->pf_eout, m->pf_ppos, m->pf_eidx, m->pf_ew, P, K, H, m->pf_x, s));
     return VVLI_OK;

@@ -1386,14 +1386,14 @@ template <int MODE, int MT, int KC, int ST, int WM, int WN, bool F32A>
 static hipError_t launch_slab_t(const GemmArgs& g, uint32_t splits, hipStream_t s) {
     using S = SlabShape<MT, KC, ST, WM, WN>;
     static const hipError_t attr =
-        hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_slab_kernel<MODE, MT, KC, ST, WM, WN, F32A>),
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_slab_kernel<MODE, MT, KC, ST, WM, WN, F32A, false>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, S::Lds);
     if (attr != hipSuccess) return attr;
     const uint32_t cols = MODE == kGemmGateUp ? 2 * g.N : g.N, tiles = (cols + kSlabN - 1) / kSlabN;
     const uint32_t items = tiles * splits;
     // Blocks take items in whole rounds: the fewest that give the same rounds.
     const uint32_t cus = gemm_cus(), rounds = (items + cus - 1) / cus;
-    return vlaunch(gemm_slab_kernel<MODE, MT, KC, ST, WM, WN, F32A>, dim3((items + rounds - 1) / rounds),
+    return vlaunch(gemm_slab_kernel<MODE, MT, KC, ST, WM, WN, F32A, false>, dim3((items + rounds - 1) / rounds),
                    dim3(kSlabThreads), S::Lds, s, g, tiles, splits);
 }
 
@@ -1500,12 +1500,32 @@ hipError_t launch_slab_reduce(const float* part, float* out, size_t n, uint32_t 
                    static_cast<uint32_t>(n), splits);
 }
 
-uint32_t grouped_gemm_tile_rows() { return kBM; }
-uint32_t grouped_gemm_max_tiles(uint32_t M, uint32_t E) { return M / kBM + E; }
+template <int MODE, int MT, int ST, int WM, int WN>
+static hipError_t launch_slab_grouped(const GemmArgs& g, hipStream_t s) {
+    using S = SlabShape<MT, 128, ST, WM, WN>;
+    constexpr int kLds = S::Lds + kSlabTable * 8;
+    static_assert(kLds <= 160 * 1024, "stages, sums and table fit");
+    static const hipError_t attr =
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_slab_kernel<MODE, MT, 128, ST, WM, WN, false, true>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+    if (attr != hipSuccess) return attr;
+    const uint32_t cols = MODE == kGemmGateUp ? 2 * g.N : g.N, tiles = (cols + kSlabN - 1) / kSlabN;
+    return vlaunch(gemm_slab_kernel<MODE, MT, 128, ST, WM, WN, false, true>, dim3(gemm_cus()), dim3(kSlabThreads), kLds,
+                   s, g, tiles, 1u);
+}
+
+// Rows of a tile by the mean rows of an expert: few rows run the few-row
+// kernel with tiles of 16 or 32, which most experts' rows fit.
+uint32_t grouped_gemm_tile_rows(uint32_t M, uint32_t E) {
+    const uint32_t rows = M <= 12 * E ? 16 : M <= 24 * E ? 32 : kBM;
+    return M / rows + E <= kSlabTable ? rows : kBM;
+}
+uint32_t grouped_gemm_max_tiles(uint32_t M, uint32_t E) { return M / grouped_gemm_tile_rows(M, E) + E; }
 
 hipError_t launch_gemm_grouped(int mode, const GemmArgs& g, hipStream_t s) {
     if (g.M == 0 || g.N == 0) return hipSuccess;
-    if (!g.a_hl || !g.tiles || g.max_tiles == 0 || g.K % 8 != 0 || (g.norm_w && !g.row_scale) ||
+    if (!g.a_hl || !g.tiles || g.max_tiles == 0 || (g.tile_rows != 16 && g.tile_rows != 32 && g.tile_rows != kBM) ||
+        (g.tile_rows != kBM && g.max_tiles > kSlabTable) || g.K % 8 != 0 || (g.norm_w && !g.row_scale) ||
         (mode != kGemmGateUp && mode != kGemmPlain) || (mode == kGemmGateUp && !g.out_hl) ||
         (mode == kGemmPlain && (g.out_hl || !g.out || g.bias[0] || g.seg_end[0] != g.N)) ||
         (g.a_plane && g.a_plane < static_cast<size_t>(g.M) * gemm_kp(g.K)) ||
@@ -1516,6 +1536,12 @@ hipError_t launch_gemm_grouped(int mode, const GemmArgs& g, hipStream_t s) {
         hipError_t e = vlaunch(gemm_split_kernel, dim3(static_cast<uint32_t>((n + 255) / 256)), dim3(256), 0, s, g);
         if (e != hipSuccess) return e;
     }
+    if (g.tile_rows == 16)
+        return mode == kGemmGateUp ? launch_slab_grouped<kGemmGateUp, 1, 6, 1, 2>(g, s)
+                                   : launch_slab_grouped<kGemmPlain, 1, 6, 1, 2>(g, s);
+    if (g.tile_rows == 32)
+        return mode == kGemmGateUp ? launch_slab_grouped<kGemmGateUp, 2, 4, 2, 1>(g, s)
+                                   : launch_slab_grouped<kGemmPlain, 2, 4, 2, 1>(g, s);
     static const hipError_t attr = [] {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_bf16_kernel<kGemmPlain, true>),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, kGemmLds);
