@@ -13,6 +13,8 @@
 //             atomics: the order over experts varies at the ulp level)
 // Every step reads the selected experts from device memory, so the token
 // step stays one replayable graph with no host round trip.
+#include <algorithm>
+
 #include "device_common.hpp"
 #include "gemv_tile.hpp"
 #include "kernels.hpp"
@@ -339,19 +341,23 @@ __global__ __launch_bounds__(kGroupThreads) void moe_group_kernel(const uint32_t
                                                                  uint32_t* __restrict__ grouped_rows,
                                                                  uint32_t* __restrict__ pair_pos,
                                                                  uint4* __restrict__ tiles) {
-    __shared__ uint8_t ids[kGroupMaxPairs];
+    __shared__ __attribute__((aligned(4))) uint8_t ids[kGroupMaxPairs];
     __shared__ uint32_t cnt[kGroupThreads];  // [g][e], then the pair offsets
     __shared__ uint32_t eoff[256], toff[257];
     const uint32_t tid = threadIdx.x;
     for (uint32_t p = tid; p < n; p += kGroupThreads) ids[p] = static_cast<uint8_t>(idx[p]);
     const uint32_t G = kGroupThreads / E;
     const uint32_t g = tid / E, e = tid % E;
-    const uint32_t span = (n + G - 1) / G;
-    const uint32_t p0 = g * span, p1 = min(n, p0 + span);
+    const uint32_t span = ((n + G - 1) / G + 3) / 4 * 4;  // whole words of ids
+    const uint32_t p0 = min(n, g * span), p1 = min(n, p0 + span);
     __syncthreads();
     uint32_t c = 0;
     if (g < G)
-        for (uint32_t p = p0; p < p1; ++p) c += ids[p] == e;
+        for (uint32_t p = p0; p < p1; p += 4) {  // (bytes past the pairs are not counted)
+            const uint32_t w = *reinterpret_cast<const uint32_t*>(ids + p);
+#pragma unroll
+            for (uint32_t q = 0; q < 4; ++q) c += p + q < p1 && ((w >> (8 * q)) & 255u) == e;
+        }
     cnt[tid] = c;
     __syncthreads();
     if (tid < E) {  // exclusive offsets over the ranges of expert tid
@@ -365,21 +371,26 @@ __global__ __launch_bounds__(kGroupThreads) void moe_group_kernel(const uint32_t
     }
     __syncthreads();
     // Totals -> offsets over experts, tile counts -> tile offsets: inclusive
-    // scans over the E entries (Hillis-Steele in LDS), made exclusive below.
-    __shared__ uint32_t scan_a[256], scan_b[256];
+    // scans over the E entries (within waves, then over the four waves' sums),
+    // made exclusive below.
+    __shared__ uint32_t scan_a[256], scan_b[256], sum_a[4], sum_b[4];
+    uint32_t va = 0, vb = 0;
     if (tid < 256) {
-        const uint32_t tot = tid < E ? eoff[tid] : 0u;
-        scan_a[tid] = tot;
-        scan_b[tid] = (tot + tile_rows - 1) / tile_rows;
+        va = tid < E ? eoff[tid] : 0u;
+        vb = (va + tile_rows - 1) / tile_rows;
+#pragma unroll
+        for (uint32_t d = 1; d < 64; d <<= 1) {
+            const uint32_t oa = __shfl_up(va, d, 64), ob = __shfl_up(vb, d, 64);
+            if ((tid & 63) >= d) va += oa, vb += ob;
+        }
+        if ((tid & 63) == 63) sum_a[tid >> 6] = va, sum_b[tid >> 6] = vb;
     }
     __syncthreads();
-    for (uint32_t d = 1; d < 256; d <<= 1) {
-        uint32_t va = 0, vb = 0;
-        if (tid < 256 && tid >= d) va = scan_a[tid - d], vb = scan_b[tid - d];
-        __syncthreads();
-        if (tid < 256) scan_a[tid] += va, scan_b[tid] += vb;
-        __syncthreads();
+    if (tid < 256) {
+        for (uint32_t w = 0; w < tid >> 6; ++w) va += sum_a[w], vb += sum_b[w];
+        scan_a[tid] = va, scan_b[tid] = vb;
     }
+    __syncthreads();
     if (tid < E) {
         const uint32_t tot = eoff[tid];
         eoff[tid] = scan_a[tid] - tot;
@@ -392,12 +403,16 @@ __global__ __launch_bounds__(kGroupThreads) void moe_group_kernel(const uint32_t
     __syncthreads();
     if (g < G) {
         uint32_t at = eoff[e] + cnt[tid];
-        for (uint32_t p = p0; p < p1; ++p)
-            if (ids[p] == e) {
-                grouped_rows[at] = p / top_k;
-                pair_pos[p] = at;
-                ++at;
-            }
+        for (uint32_t p = p0; p < p1; p += 4) {
+            const uint32_t w = *reinterpret_cast<const uint32_t*>(ids + p);
+#pragma unroll
+            for (uint32_t q = 0; q < 4; ++q)
+                if (p + q < p1 && ((w >> (8 * q)) & 255u) == e) {
+                    grouped_rows[at] = (p + q) / top_k;
+                    pair_pos[p + q] = at;
+                    ++at;
+                }
+        }
     }
     if (tid < E) {
         const uint32_t b = eoff[tid], end = tid + 1 < E ? eoff[tid + 1] : n;
@@ -406,33 +421,30 @@ __global__ __launch_bounds__(kGroupThreads) void moe_group_kernel(const uint32_t
     }
 }
 
-// One block per row: its (expert, weight, grouped position) triples sorted
-// by expert id in LDS, then x[r][i] += sum_j eout[pos_j][i] * w_j in that
+// Blocks of a row's columns: its (weight, grouped position) pairs in expert
+// order in LDS, then x[r][i] += sum_j eout[pos_j][i] * w_j in that
 // order (products rounded, then added: the oracle's moe += out * w).
 __global__ __launch_bounds__(kThreads) void moe_combine_kernel(const float* __restrict__ eout,
                                                               const uint32_t* __restrict__ pair_pos,
                                                               const uint32_t* __restrict__ idx,
                                                               const float* __restrict__ weight, uint32_t top_k,
                                                               uint32_t H, float* __restrict__ x) {
-    __shared__ uint32_t se[kMaxTopK], sp[kMaxTopK];
+    __shared__ uint32_t sp[kMaxTopK];
     __shared__ float sw[kMaxTopK];
     const uint32_t r = blockIdx.x;
-    if (threadIdx.x == 0) {
-        for (uint32_t j = 0; j < top_k; ++j) {  // insertion sort by expert id (ids of a row are distinct)
-            const size_t p = static_cast<size_t>(r) * top_k + j;
-            const uint32_t ej = idx[p], pj = pair_pos[p];
-            const float wj = weight[p];
-            uint32_t k = j;
-            while (k > 0 && se[k - 1] > ej) {
-                se[k] = se[k - 1], sp[k] = sp[k - 1], sw[k] = sw[k - 1];
-                --k;
-            }
-            se[k] = ej, sp[k] = pj, sw[k] = wj;
-        }
+    if (threadIdx.x < top_k) {  // slot j goes to the rank of its expert id (a row's ids are distinct)
+        const uint32_t* ids = idx + static_cast<size_t>(r) * top_k;
+        const size_t p = static_cast<size_t>(r) * top_k + threadIdx.x;
+        const uint32_t mine = ids[threadIdx.x], at = pair_pos[p];
+        const float w = weight[p];
+        uint32_t rank = 0;
+#pragma unroll
+        for (uint32_t j = 0; j < static_cast<uint32_t>(kMaxTopK); ++j) rank += j < top_k && ids[j < top_k ? j : 0] < mine;
+        sp[rank] = at, sw[rank] = w;
     }
     __syncthreads();
     float* xr = x + static_cast<size_t>(r) * H;
-    for (uint32_t i = threadIdx.x; i < H; i += kThreads) {
+    for (uint32_t i = blockIdx.y * kThreads + threadIdx.x; i < H; i += gridDim.y * kThreads) {
         float v[kMaxTopK];  // every slot's load in flight before the ordered sum
 #pragma unroll
         for (int j = 0; j < kMaxTopK; ++j)
@@ -468,7 +480,9 @@ hipError_t launch_moe_combine(const float* eout, const uint32_t* pair_pos, const
                               uint32_t rows, uint32_t top_k, uint32_t H, float* x, hipStream_t s) {
     if (rows == 0) return hipSuccess;
     if (top_k == 0 || top_k > static_cast<uint32_t>(kMaxTopK)) return hipErrorInvalidValue;
-    return vlaunch(moe_combine_kernel, dim3(rows), dim3(kThreads), 0, s, eout, pair_pos, idx, weight, top_k, H, x);
+    // Few rows: their columns over several blocks.
+    const uint32_t cols = rows <= 256 ? std::min(4u, (H + kThreads - 1) / kThreads) : 1u;
+    return vlaunch(moe_combine_kernel, dim3(rows, cols), dim3(kThreads), 0, s, eout, pair_pos, idx, weight, top_k, H, x);
 }
 
 hipError_t moe_gemv_init_attributes() {
