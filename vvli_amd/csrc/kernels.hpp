@@ -448,7 +448,9 @@ struct PrefillAttnArgs {
 // cache rows (0 for an unsupported head_dim).
 size_t prefill_kv_pack_bytes(uint32_t keys, uint32_t kv_heads, uint32_t hd);
 hipError_t launch_prefill_attn(const PrefillAttnArgs& a, uint32_t hd, hipStream_t s);
-// The same in f32 throughout (prefill_f32.hip; head_dim 32, 64 or 128).
+// The same in f32 throughout, from the cache rows (prefill_f32.hip; head_dim
+// 32, 64 or 128), and whether a prompt of bf16 weights is short enough for it.
+bool attn_f32_short(uint32_t rows, uint32_t start, uint32_t heads, uint32_t hd);
 hipError_t launch_attn_f32(const PrefillAttnArgs& a, uint32_t hd, hipStream_t s);
 // false (default): the MFMA flash-attention kernel; true: the f32 vector kernel.
 extern bool prefill_attn_vector;

@@ -16,6 +16,7 @@ namespace vvli {
 namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 
 // ---------------------------------------------------------------------------
 // out[M][N] = A[M][K] . W[N][K]^T.
@@ -340,8 +341,21 @@ __global__ __launch_bounds__(kF32Threads) void attn_f32_kernel(PrefillAttnArgs a
         f32x4 r = so[0][d][lane] * wt[0];
 #pragma unroll
         for (int w = 1; w < kF32Waves; ++w) r += so[w][d][lane] * wt[w];
-        if (v0 + fr < nvec)
-            *reinterpret_cast<f32x4*>(a.out + static_cast<size_t>(row) * a.ldo + head * HD + d * 16 + fq * 4) = r * inv;
+        if (v0 + fr >= nvec) continue;
+        r *= inv;
+        if (a.out_hl) {  // split planes of o_proj's A: hi = bf16(x), lo = bf16(x - hi)
+            bf16x4 hi, lo;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                hi[e] = static_cast<__bf16>(r[e]);
+                lo[e] = static_cast<__bf16>(r[e] - static_cast<float>(hi[e]));
+            }
+            uint16_t* hp = a.out_hl + static_cast<size_t>(row) * (a.heads * HD) + head * HD + d * 16 + fq * 4;
+            *reinterpret_cast<bf16x4*>(hp) = hi;
+            *reinterpret_cast<bf16x4*>(hp + a.out_plane) = lo;
+        } else {
+            *reinterpret_cast<f32x4*>(a.out + static_cast<size_t>(row) * a.ldo + head * HD + d * 16 + fq * 4) = r;
+        }
     }
 }
 
@@ -404,9 +418,23 @@ hipError_t launch_embed_rows_f32(const float* embed, const uint32_t* tokens, uin
     return vlaunch(embed_rows_f32_kernel, dim3((n / 4 + 255) / 256, rows), dim3(256), 0, s, embed, tokens, n, x);
 }
 
+// Whether bf16 prompts take it: the MFMA attention of prefill.hip does three
+// bf16 products for each f32 one here, about five times as fast, but wants its
+// K/V tile images written first (a pass over the earlier rows, scattered
+// stores for the new ones) and runs 64 vectors a block. Whole prompts, us a
+// layer, that / this: 1B shape 45 rows after 200 94 / 88, 64 after 2000 138 /
+// 119, 256 after 500 160 / 157, 400 201 / 198, 512 210 / 212; Qwen2.5-0.5B 32
+// rows 63 / 60, 400 after 300 135 / 128, 700 141 / 141; OLMoE 256 391 / 380.
+bool attn_f32_short(uint32_t rows, uint32_t start, uint32_t heads, uint32_t hd) {
+    const float pairs = static_cast<float>(heads) * rows * (start + 0.5f * rows) * (hd / 64.f);
+    return pairs <= (start ? 6e6f : 3e6f);
+}
+
 hipError_t launch_attn_f32(const PrefillAttnArgs& a, uint32_t hd, hipStream_t s) {
     if (a.rows == 0) return hipSuccess;
-    if (a.kv_heads == 0 || a.heads % a.kv_heads != 0 || a.out_hl) return hipErrorInvalidValue;
+    if (a.kv_heads == 0 || a.heads % a.kv_heads != 0 ||
+        (a.out_hl && (a.out_plane < static_cast<size_t>(a.rows) * a.heads * hd)))
+        return hipErrorInvalidValue;
     const uint32_t G = a.heads / a.kv_heads;
     const dim3 grid((a.rows * G + 15) / 16 * a.kv_heads);
     switch (hd) {
