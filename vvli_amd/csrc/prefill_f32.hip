@@ -5,7 +5,10 @@
 // shared; the norm, the matrix products and the attention are here.
 //
 // The token loop reads all weights once per token: Qwen2.5-0.5B's layers at 48
-// rows (four of them, 240 MB) took 10.05 ms, 209 us a token.
+// rows (four of them, 240 MB) took 10.05 ms, 209 us a token; here 326 us. What
+// bounds them now is latency: eight launches a layer of 3.5 to 25 us (gate/up 25,
+// o_proj and down 9 on average, q|k|v 7; gate/up's bytes and products take 6
+// each), with two of a block's load groups in flight.
 #include <algorithm>
 
 #include "device_common.hpp"
@@ -47,8 +50,8 @@ __device__ __forceinline__ const float* f32_w_row(const F32GemmArgs& g, uint32_t
 
 template <int MODE, int MT, int NT, int U>
 __global__ __launch_bounds__(kF32Threads, 2) void gemm_f32_kernel(F32GemmArgs g, uint32_t tm, uint32_t tn) {
-    static_assert(MODE != kGemmGateUp || NT == 2, "a gate tile and its up tile");
-    constexpr int NOut = MODE == kGemmGateUp ? 16 : NT * 16;  // output columns of a block
+    // GateUp: the W rows of a 16-column tile are 8 gate rows and their 8 up rows.
+    constexpr int NOut = MODE == kGemmGateUp ? NT * 8 : NT * 16;  // output columns of a block
     __shared__ f32x4 red[kF32Waves][MT * NT][64];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -72,8 +75,10 @@ __global__ __launch_bounds__(kF32Threads, 2) void gemm_f32_kernel(F32GemmArgs g,
         pa[i] = g.a + static_cast<size_t>(min(m0 + i * 16 + fr, g.M - 1)) * g.lda;
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
-        if (MODE == kGemmGateUp) pw[j] = (j ? g.w_up : g.w[0]) + static_cast<size_t>(n0 + fr < g.N ? n0 + fr : 0) * g.K;
-        else pw[j] = f32_w_row(g, n0 + j * 16 + fr);
+        if (MODE == kGemmGateUp) {
+            const uint32_t n = n0 + j * 8 + (fr & 7);
+            pw[j] = (fr < 8 ? g.w[0] : g.w_up) + static_cast<size_t>(n < g.N ? n : 0) * g.K;
+        } else pw[j] = f32_w_row(g, n0 + j * 16 + fr);
     }
     f32x4 sum[MT][NT];
 #pragma unroll
@@ -147,27 +152,27 @@ __global__ __launch_bounds__(kF32Threads, 2) void gemm_f32_kernel(F32GemmArgs g,
     const bool split = gridDim.z > 1;
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
-        if (MODE == kGemmGateUp) {
-            if (i % kF32Waves != wave) continue;
-            f32x4 gt = red[0][2 * i][lane], up = red[0][2 * i + 1][lane];
-#pragma unroll
-            for (int w = 1; w < kF32Waves; ++w) gt += red[w][2 * i][lane], up += red[w][2 * i + 1][lane];
-            const uint32_t n = n0 + fr;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const uint32_t row = m0 + i * 16 + 4 * fq + e;
-                if (row < g.M && n < g.N)  // siluMulInto, src/llm.zig:1382-1387
-                    g.out[static_cast<size_t>(row) * g.ldo + n] =
-                        __fmul_rn(__fdiv_rn(gt[e], __fadd_rn(1.0f, expf(-gt[e]))), up[e]);
-            }
-            continue;
-        }
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
             if ((i * NT + j) % kF32Waves != wave) continue;
             f32x4 v = red[0][i * NT + j][lane];
 #pragma unroll
             for (int w = 1; w < kF32Waves; ++w) v += red[w][i * NT + j][lane];
+            if (MODE == kGemmGateUp) {  // the up sums sit eight lanes on
+                const int up_lane = (lane & ~15) + 8 + (lane & 7);
+                f32x4 up = red[0][i * NT + j][up_lane];
+#pragma unroll
+                for (int w = 1; w < kF32Waves; ++w) up += red[w][i * NT + j][up_lane];
+                const uint32_t n = n0 + j * 8 + fr;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const uint32_t row = m0 + i * 16 + 4 * fq + e;
+                    if (fr < 8 && row < g.M && n < g.N)  // siluMulInto, src/llm.zig:1382-1387
+                        g.out[static_cast<size_t>(row) * g.ldo + n] =
+                            __fmul_rn(__fdiv_rn(v[e], __fadd_rn(1.0f, expf(-v[e]))), up[e]);
+                }
+                continue;
+            }
             const uint32_t n = n0 + j * 16 + fr;
             if (n >= g.N) continue;
             float bias = 0.f;
@@ -361,31 +366,35 @@ __global__ __launch_bounds__(kF32Threads) void attn_f32_kernel(PrefillAttnArgs a
 
 template <int MODE, int MT, int NT, int U>
 hipError_t launch_t(const F32GemmArgs& g, uint32_t splits, hipStream_t s) {
-    const uint32_t nout = MODE == kGemmGateUp ? 16 : NT * 16;
+    const uint32_t nout = MODE == kGemmGateUp ? NT * 8 : NT * 16;
     const uint32_t tm = (g.M + MT * 16 - 1) / (MT * 16), tn = (g.N + nout - 1) / nout;
     return vlaunch(gemm_f32_kernel<MODE, MT, NT, U>, dim3(tm * tn, 1, splits), dim3(kF32Threads), 0, s, g, tm, tn);
 }
 
+// Tiles and steps in flight: one 16-column tile of W a block up to 64 rows (two
+// where gate and up share a block), few steps a buffer so that several blocks
+// share a CU. 48 rows through four Qwen2.5-0.5B layers 375 -> 326 us against
+// four steps and at least eight a wave.
 template <int MODE>
 hipError_t launch_mode(const F32GemmArgs& g, uint32_t splits, hipStream_t s) {
     constexpr int NT = MODE == kGemmGateUp ? 2 : 1;
-    if (g.M <= 16) return launch_t<MODE, 1, NT, 4>(g, splits, s);
-    if (g.M <= 32) return launch_t<MODE, 2, NT, 4>(g, splits, s);
-    if (g.M <= 48) return launch_t<MODE, 3, NT, NT == 1 ? 4 : 2>(g, splits, s);
-    if (g.M <= 64) return launch_t<MODE, 4, NT, NT == 1 ? 4 : 2>(g, splits, s);
-    return launch_t<MODE, 4, 2, 2>(g, splits, s);
+    if (g.M <= 16) return launch_t<MODE, 1, NT, 2>(g, splits, s);
+    if (g.M <= 32) return launch_t<MODE, 2, NT, 2>(g, splits, s);
+    if (g.M <= 48) return launch_t<MODE, 3, NT, 1>(g, splits, s);
+    if (g.M <= 64) return launch_t<MODE, 4, NT, 1>(g, splits, s);
+    return launch_t<MODE, 4, 2, 1>(g, splits, s);
 }
 
 }  // namespace
 
 // K splits (Plain and Resid, with `part`): up to two blocks per CU, each wave
-// of a split at least 8 K steps, at most kMaxPartSplits.
+// of a split at least 2 K steps, at most kMaxPartSplits.
 uint32_t gemm_f32_splits(int mode, const F32GemmArgs& g) {
     if (mode == kGemmGateUp || !g.part) return 1;
     const uint32_t mt = g.M <= 16 ? 1 : g.M <= 32 ? 2 : g.M <= 48 ? 3 : 4, nt = g.M <= 64 ? 1 : 2;
     const uint32_t tiles = ((g.M + mt * 16 - 1) / (mt * 16)) * ((g.N + nt * 16 - 1) / (nt * 16));
     const uint32_t nk = (g.K + 15) / 16;
-    uint32_t splits = std::max(1u, std::min({512u / std::max(1u, tiles), nk / (kF32Waves * 8), kMaxPartSplits}));
+    uint32_t splits = std::max(1u, std::min({512u / std::max(1u, tiles), nk / (kF32Waves * 2), kMaxPartSplits}));
     while (splits > 1 && static_cast<size_t>(splits) * g.M * g.N > gemm_part_elems()) --splits;
     const uint32_t per = (nk + splits - 1) / splits;
     return (nk + per - 1) / per;  // every split gets K steps
