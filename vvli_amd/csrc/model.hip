@@ -765,8 +765,11 @@ int ensure_prefill_buffers(vvli_gpu_model* m);
 bool use_batched_prefill(vvli_gpu_model* m) {
     if (m->prefill_path == 1) return false;
     if (prefill_supported(m->cfg)) return true;
-    // (the token loop needs no chunk buffers: it serves where they do not fit)
-    return prefill_f32_supported(m->cfg) && ensure_prefill_buffers(m) == VVLI_OK;
+    // The token loop needs no chunk buffers: it serves where they do not fit.
+    if (!prefill_f32_supported(m->cfg) || hipSetDevice(m->device) != hipSuccess) return false;
+    if (ensure_prefill_buffers(m) == VVLI_OK) return true;
+    (void)hipGetLastError();  // (else the loop's first launch would report it)
+    return false;
 }
 
 int ensure_prefill_buffers(vvli_gpu_model* m) {
