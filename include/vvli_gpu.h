@@ -364,6 +364,17 @@ int vvli_gpu_linear(const uint16_t* dW, const float* dX, const uint16_t* dBias, 
 int vvli_gpu_linear_noalloc(const uint16_t* dW, const float* dX, const uint16_t* dBias, float* dY, uint32_t M,
                             uint32_t N, uint32_t K, void* stream);
 
+/* Test hook of vvli_gpu_linear (no reference counterpart; needs no GPU): what
+ * a call with 16-byte aligned dW and dX runs on a device of `cus` compute
+ * units. kernel: 0 GEMV, 1 skinny, 2 few-row GEMM, 3 tiles; splits: of K;
+ * gemm_few_rows: whether the prefill GEMM, given these sizes, would run its
+ * few-row kernel; scratch_bytes: scratch of the call (0: none). */
+typedef struct vvli_gpu_linear_route {
+    uint32_t kernel, splits, gemm_few_rows, reserved;
+    uint64_t scratch_bytes;
+} vvli_gpu_linear_route;
+int vvli_gpu_test_linear_route(uint32_t M, uint32_t N, uint32_t K, uint32_t cus, vvli_gpu_linear_route* out);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,0 +1,36 @@
+"""Which kernel vvli_gpu_linear runs, from the sizes and the device's compute
+units alone (host arithmetic: no GPU)."""
+import pytest
+
+from vvli_amd import runtime as R
+
+SIZES = [(2048, 2048), (8192, 2048), (16384, 2048), (4096, 2048), (2048, 8192), (3584, 18944), (18944, 3584),
+         (128256, 2048), (130, 72), (200, 40), (2048, 8)]
+ROWS = [1, 2, 3, 4, 5, 16, 17, 33, 64, 65, 96, 100, 127, 128, 129, 512]
+
+
+def kernel(route) -> str:
+    return R.LINEAR_KERNELS[route.kernel]
+
+
+@pytest.mark.parametrize("cus", [32, 64, 128, 192, 256, 304])
+def test_few_rows_only_where_the_gemm_takes_it(cus):
+    """A call that is planned without split planes runs the few-row kernel, and
+    the others above 64 rows have room for their planes: whatever the number
+    of compute units (a partitioned device, a mask), the GEMM's own plan is the
+    one that decides."""
+    for M in ROWS:
+        for N, K in SIZES:
+            r = R.linear_route(M, N, K, cus)
+            if kernel(r) == "few_rows":
+                assert r.gemm_few_rows and M <= 128, (M, N, K, cus)
+            elif M > 64:
+                assert kernel(r) == "tiles" and r.scratch_bytes >= 4 * M * K, (M, N, K, cus)
+                assert M > 128 or not r.gemm_few_rows, (M, N, K, cus)
+
+
+def test_few_rows_past_one_round_of_a_small_device():
+    # 256 and 64 items of 64 rows of W: one round of 256 CUs, more than one of 128 and of 32.
+    assert kernel(R.linear_route(128, 16384, 2048, 256)) == "few_rows"
+    assert kernel(R.linear_route(128, 16384, 2048, 128)) == "tiles"
+    assert kernel(R.linear_route(100, 4096, 2048, 32)) == "tiles"

@@ -92,6 +92,16 @@ class CSampling(ctypes.Structure):
     ]
 
 
+class CLinearRoute(ctypes.Structure):
+    _fields_ = [
+        ("kernel", c_uint32),
+        ("splits", c_uint32),
+        ("gemm_few_rows", c_uint32),
+        ("reserved", c_uint32),
+        ("scratch_bytes", c_uint64),
+    ]
+
+
 # void (*)(void* user, size_t completed, size_t total, const char* name)
 PROGRESS_FN = ctypes.CFUNCTYPE(None, c_void_p, c_size_t, c_size_t, c_char_p)
 
@@ -146,6 +156,7 @@ PROTOTYPES = {
     "vvli_gpu_linear": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_uint32, c_uint32, c_uint32, c_void_p]),
     "vvli_gpu_linear_noalloc": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_uint32, c_uint32, c_uint32,
                                         c_void_p]),
+    "vvli_gpu_test_linear_route": (c_int, [c_uint32, c_uint32, c_uint32, c_uint32, POINTER(CLinearRoute)]),
     "vvli_host_fill_deterministic": (None, [c_void_p, c_size_t, c_uint32]),
     "vvli_host_fill_synthetic": (c_int, [POINTER(CConfig), c_uint64, c_float, c_void_p, c_size_t, c_uint32]),
     "vvli_host_synthetic_normal": (c_double, [c_uint64, c_uint64, c_uint64]),

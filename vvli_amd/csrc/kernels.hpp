@@ -336,14 +336,21 @@ struct GemmArgs {
 // kernel splits only launches that are given `part`), and the
 // capacity of the partial sums buffer any launch needs (elements).
 uint32_t gemm_splits(int mode, const GemmArgs& g);
-// gemm_splits of a dense Plain launch that is given `part`.
-uint32_t gemm_plain_part_splits(uint32_t M, uint32_t N, uint32_t K);
+uint32_t gemm_cus();  // CUs of the device
 size_t gemm_part_elems();
-// The few-row kernel (M <= kSlabMaxRows): the splits it uses for a Plain launch
-// that is given `part`. launch_slab_reduce adds up any Plain launch's splits:
-// out[i] = sum of part[z * n + i].
-constexpr uint32_t kSlabMaxRows = 128;
-uint32_t gemm_slab_part_splits(uint32_t M, uint32_t N, uint32_t K);
+// What a dense Plain launch that is given `part` runs on a device of `cus` CUs:
+// the few-row kernel or tiles, and its K splits.
+constexpr uint32_t kSlabMaxRows = 128;  // most rows of the few-row kernel
+struct PlainGemmPlan {
+    bool few_rows;
+    uint32_t splits;
+};
+PlainGemmPlan gemm_plain_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t cus);
+// The few-row kernel on f32 rows of A, which it splits itself (one segment of
+// W; a and W 16-byte aligned): `splits` as gemm_plain_plan gives them, `part`
+// needed where they are more than one. launch_slab_reduce adds up any Plain
+// launch's splits: out[i] = sum of part[z * n + i].
+hipError_t launch_gemm_few_rows(const GemmArgs& g, uint32_t splits, hipStream_t s);
 hipError_t launch_slab_reduce(const float* part, float* out, size_t n, uint32_t splits, hipStream_t s);
 __host__ __device__ inline uint32_t gemm_kp(uint32_t K) { return (K + 31) / 32 * 32; }
 size_t gemm_split_elems(uint32_t M, uint32_t K);

@@ -22,8 +22,8 @@ namespace {
 // Rows from which one MFMA kernel replaces the GEMV kernel (linear_gemv.hpp,
 // up to 4 rows of x in one launch: 4 only where the skinny kernel would split
 // K across blocks, linear_uses_gemv); up to kSkinnyMaxRows the skinny kernel
-// below or the few-row GEMM (gemm_slab.hpp, up to kSlabMaxRows; linear_uses_slab),
-// beyond it the prefill GEMM.
+// below or the few-row GEMM (gemm_slab.hpp, up to kSlabMaxRows), beyond it the
+// prefill GEMM's tiles (linear_plan).
 constexpr uint32_t kLinearGemmMinRows = 4;
 constexpr uint32_t kSkinnyMaxRows = 64;
 
@@ -390,85 +390,92 @@ bool linear_uses_gemv(uint32_t M, uint32_t N, uint32_t K) {
 // skinny kernel moves about 40 KB per us; a chunk of the few-row GEMM takes
 // kChunkUs. Measured, skinny / few-row: 2048 x 8192 M = 16 22.2 / 11.4, M = 64
 // 44.7 / 16.0; 128256 x 2048 M = 16 132.7 / 96; 2048 x 2048 M = 8 6.4 / 7.7,
-// M = 33 12.8 / 9.5; 1152 x 896 M = 33 7.0 / 8.0. From 65 to 128 rows against
-// the split pass and the 128 x 256 tiles: the few-row GEMM while its items are
-// one round (2048 x 2048 M = 96 21.8 / 13.7; 8192 x 2048 M = 128 34.7 / 25.5),
-// the tiles beyond (18944 x 3584 M = 128 61 / 102).
-bool slab_beats_skinny(uint32_t M, uint32_t N, uint32_t K) {
+// M = 33 12.8 / 9.5; 1152 x 896 M = 33 7.0 / 8.0. From 65 to 128 rows what
+// gemm_plain_plan takes, against the split pass and the tiles: 2048 x 2048 M =
+// 96 21.8 / 13.7; 8192 x 2048 M = 128 34.7 / 25.5.
+bool slab_beats_skinny(uint32_t M, uint32_t N, uint32_t K, uint32_t slab_splits, uint32_t cus) {
     const float rows = static_cast<float>(M), k = static_cast<float>(K);
     const uint32_t ks0 = skinny_splits(N, K), blocks = skinny_tiles(N) * ks0;
     const float skinny = 2.8f + (ks0 > 1 ? 5.f : 0.f) +
-                         static_cast<float>((blocks + 255) / 256) * (k / ks0) * (4.f * rows + 32.f * skinny_nt(N)) / 40e3f;
+                         static_cast<float>((blocks + cus - 1) / cus) * (k / ks0) * (4.f * rows + 32.f * skinny_nt(N)) / 40e3f;
     constexpr float kChunkUs[] = {0.5f, 0.65f, 0.95f, 0.95f};  // 16, 32, 64 rows
-    const uint32_t ks = gemm_slab_part_splits(M, N, K), tiles = (N + 63) / 64, chunks = ((K + 127) / 128 + ks - 1) / ks;
+    const uint32_t ks = slab_splits, tiles = (N + 63) / 64, chunks = ((K + 127) / 128 + ks - 1) / ks;
     const float slab = 4.4f + (ks > 1 ? 2.6f : 0.f) +
-                       static_cast<float>((tiles * ks + 255) / 256 * chunks) * kChunkUs[(M - 1) / 16];
+                       static_cast<float>((tiles * ks + cus - 1) / cus * chunks) * kChunkUs[(M - 1) / 16];
     return slab < skinny;
 }
 
-bool linear_uses_slab(const uint16_t* dW, const float* dX, uint32_t M, uint32_t N, uint32_t K) {
-    if (M < kLinearGemmMinRows || M > kSlabMaxRows || linear_uses_gemv(M, N, K) ||
-        (reinterpret_cast<uintptr_t>(dW) | reinterpret_cast<uintptr_t>(dX)) % 16 != 0)
-        return false;
-    return M <= kSkinnyMaxRows ? slab_beats_skinny(M, N, K) : (N + 63) / 64 * gemm_slab_part_splits(M, N, K) <= 256;
-}
+// What a call runs, from its sizes and the device's CUs alone.
+enum class LinearKernel : uint32_t { Gemv, Skinny, FewRows, Tiles };
+struct LinearPlan {
+    LinearKernel kernel = LinearKernel::Gemv;
+    uint32_t splits = 1;  // K splits (Tiles: added atomically unless part > 0)
+    size_t payload = 0;   // Skinny, FewRows: K-split partials; Tiles: the split planes
+    size_t part = 0;      // Tiles: K-split partials behind the planes
+    size_t bytes() const { return payload ? kCounterBytes + payload + part : 0; }
+};
 
-// M > 64: the split planes, and behind them the partial sums of a K split
-// (0: the launch does not split K, or more ways than the summing pass takes).
 size_t linear_plane_bytes(uint32_t M, uint32_t K) { return gemm_split_elems(M, K) * sizeof(uint16_t); }
-size_t linear_part_bytes(uint32_t M, uint32_t N, uint32_t K) {
-    if (M <= kSkinnyMaxRows) return 0;
-    const uint32_t ks = gemm_plain_part_splits(M, N, K);
-    return ks > 1 && ks <= 8 ? (size_t)ks * M * N * sizeof(float) : 0;
+
+// aligned: W and X are at 16-byte addresses. lean: without partial sums, as a
+// call that cannot have more scratch runs.
+LinearPlan linear_plan(uint32_t M, uint32_t N, uint32_t K, bool aligned, bool lean, uint32_t cus) {
+    LinearPlan p;
+    if (linear_uses_gemv(M, N, K)) return p;
+    const size_t sums = (size_t)M * N * sizeof(float);
+    if (M <= kSlabMaxRows && aligned && !lean) {
+        const PlainGemmPlan g = gemm_plain_plan(M, N, K, cus);
+        if (g.few_rows && (M > kSkinnyMaxRows || slab_beats_skinny(M, N, K, g.splits, cus))) {
+            p.kernel = LinearKernel::FewRows, p.splits = g.splits;
+            p.payload = g.splits > 1 ? g.splits * sums : 0;
+            return p;
+        }
+    }
+    if (M <= kSkinnyMaxRows) {
+        p.kernel = LinearKernel::Skinny, p.splits = skinny_splits(N, K);
+        p.payload = p.splits > 1 ? p.splits * sums : 0;
+        return p;
+    }
+    p.kernel = LinearKernel::Tiles, p.payload = linear_plane_bytes(M, K);
+    if (!lean) {  // (the summing pass takes up to 8 splits)
+        p.splits = gemm_plain_plan(M, N, K, cus).splits;
+        if (p.splits > 1 && p.splits <= 8) p.part = p.splits * sums;
+    }
+    return p;
 }
 
-size_t linear_payload_bytes(bool slab, uint32_t M, uint32_t N, uint32_t K) {
-    if (slab) {
-        const uint32_t ks = gemm_slab_part_splits(M, N, K);
-        return ks > 1 ? (size_t)ks * M * N * sizeof(float) : 0;
-    }
-    if (M > kSkinnyMaxRows) return linear_plane_bytes(M, K);
-    if (linear_uses_gemv(M, N, K)) return 0;
-    if (M >= kLinearGemmMinRows) {
-        const uint32_t ks = skinny_splits(N, K);
-        return ks > 1 ? (size_t)ks * M * N * sizeof(float) : 0;
-    }
-    return 0;
+LinearPlan linear_plan(const uint16_t* dW, const float* dX, uint32_t M, uint32_t N, uint32_t K, bool lean = false) {
+    const bool aligned = (reinterpret_cast<uintptr_t>(dW) | reinterpret_cast<uintptr_t>(dX)) % 16 == 0;
+    return linear_plan(M, N, K, aligned, lean, gemm_cus());
 }
 
-// Enqueue the op on s. scratch: kCounterBytes + linear_payload_bytes of
-// device memory laid out as above (and linear_part_bytes behind them with
-// `parts`: else the splits add atomically), or null when the payload is 0.
-int linear_enqueue(bool slab, bool parts, const uint16_t* dW, const float* dX, const uint16_t* dBias, float* dY, uint32_t M,
+// Enqueue the op on s. scratch: p.bytes() of device memory laid out as above
+// (null when that is 0).
+int linear_enqueue(const LinearPlan& p, const uint16_t* dW, const float* dX, const uint16_t* dBias, float* dY, uint32_t M,
                    uint32_t N, uint32_t K, hipStream_t s, char* scratch_mem) {
-    if (slab) {
-        const uint32_t ks = gemm_slab_part_splits(M, N, K);
-        GemmArgs g;
-        g.a = dX, g.lda = K, g.w[0] = dW, g.bias[0] = dBias;
-        g.seg_end[0] = g.seg_end[1] = g.seg_end[2] = N;
-        g.out = dY, g.ldo = N, g.M = M, g.N = N, g.K = K;
-        if (ks > 1) g.part = reinterpret_cast<float*>(scratch_mem + kCounterBytes);
-        HIP_TRY(launch_gemm_bf16(kGemmPlain, g, s));
-        if (ks > 1) HIP_TRY(launch_slab_reduce(g.part, dY, (size_t)M * N, ks, s));
-        return VVLI_OK;
-    }
-    if (M >= kLinearGemmMinRows && M <= kSkinnyMaxRows && !linear_uses_gemv(M, N, K)) {
+    if (p.kernel == LinearKernel::Skinny) {
         float* ws = scratch_mem ? reinterpret_cast<float*>(scratch_mem + kCounterBytes) : nullptr;
         uint32_t* cnt = reinterpret_cast<uint32_t*>(scratch_mem);
         HIP_TRY(launch_skinny(dW, dX, dBias, dY, M, N, K, ws, cnt, s));
         return VVLI_OK;
     }
-    if (M > kSkinnyMaxRows) {
-        // One MFMA GEMM reads W once for all rows; the activations are split
-        // hi/lo into a_hl first.
+    if (p.kernel == LinearKernel::FewRows || p.kernel == LinearKernel::Tiles) {
         GemmArgs g;
         g.a = dX, g.lda = K, g.w[0] = dW, g.bias[0] = dBias;
         g.seg_end[0] = g.seg_end[1] = g.seg_end[2] = N;
         g.out = dY, g.ldo = N, g.M = M, g.N = N, g.K = K;
-        g.a_hl = reinterpret_cast<uint16_t*>(scratch_mem + kCounterBytes);
-        if (parts) g.part = reinterpret_cast<float*>(scratch_mem + kCounterBytes + linear_plane_bytes(M, K));
-        HIP_TRY(launch_gemm_bf16(kGemmPlain, g, s));
-        if (parts) HIP_TRY(launch_slab_reduce(g.part, dY, (size_t)M * N, gemm_splits(kGemmPlain, g), s));
+        char* const payload = scratch_mem + kCounterBytes;
+        if (p.kernel == LinearKernel::FewRows) {
+            if (p.splits > 1) g.part = reinterpret_cast<float*>(payload);
+            HIP_TRY(launch_gemm_few_rows(g, p.splits, s));
+        } else {
+            // One MFMA GEMM reads W once for all rows; the activations are
+            // split hi/lo into a_hl first.
+            g.a_hl = reinterpret_cast<uint16_t*>(payload);
+            if (p.part) g.part = reinterpret_cast<float*>(payload + p.payload);
+            HIP_TRY(launch_gemm_bf16(kGemmPlain, g, s));
+        }
+        if (g.part) HIP_TRY(launch_slab_reduce(g.part, dY, (size_t)M * N, p.splits, s));
         return VVLI_OK;
     }
     // M <= 4: one GEMV launch for all rows when their x fits LDS, else one per row.
@@ -513,12 +520,8 @@ int vvli_gpu_linear(const uint16_t* dW, const float* dX, const uint16_t* dBias, 
     int rc = check_linear_args(dW, dX, dY, M, N, K, "vvli_gpu_linear");
     if (rc) return rc;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    bool slab = linear_uses_slab(dW, dX, M, N, K);
-    size_t payload = linear_payload_bytes(slab, M, N, K);
-    if (payload == 0) return linear_enqueue(slab, false, dW, dX, dBias, dY, M, N, K, s, nullptr);
-    const size_t part_bytes = slab ? 0 : linear_part_bytes(M, N, K);
-    bool parts = part_bytes > 0;
-    size_t need = kCounterBytes + payload + part_bytes;
+    LinearPlan p = linear_plan(dW, dX, M, N, K);
+    if (p.bytes() == 0) return linear_enqueue(p, dW, dX, dBias, dY, M, N, K, s, nullptr);
     // The scratch is kept per stream and grows stream-ordered (its counters
     // cleared once per allocation); the lock covers the enqueue, so calls on
     // one stream use it in turn.
@@ -537,45 +540,54 @@ int vvli_gpu_linear(const uint16_t* dW, const float* dX, const uint16_t* dBias, 
         cache.push_back(StreamScratch{s, nullptr, 0});
         sc = &cache.back();
     }
-    if ((slab || parts) && sc->bytes < need) {
+    if (sc->bytes < p.bytes() && (p.kernel == LinearKernel::FewRows || p.part > 0)) {
         // Under stream capture nothing may be allocated for a call that the
         // other kernels serve without scratch or with less: they take it.
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
             (void)hipGetLastError();
-            slab = parts = false;
-            payload = linear_payload_bytes(slab, M, N, K);
-            if (payload == 0) return linear_enqueue(slab, parts, dW, dX, dBias, dY, M, N, K, s, nullptr);
-            need = kCounterBytes + payload;
+            p = linear_plan(dW, dX, M, N, K, true);
+            if (p.bytes() == 0) return linear_enqueue(p, dW, dX, dBias, dY, M, N, K, s, nullptr);
         }
     }
-    if (sc->bytes < need) {
+    if (sc->bytes < p.bytes()) {
         if (sc->p) HIP_TRY(hipFreeAsync(sc->p, s));
         sc->p = nullptr, sc->bytes = 0;
-        HIP_TRY(hipMallocAsync(&sc->p, need, s));
+        HIP_TRY(hipMallocAsync(&sc->p, p.bytes(), s));
         HIP_TRY(hipMemsetAsync(sc->p, 0, kCounterBytes, s));
-        sc->bytes = need;
+        sc->bytes = p.bytes();
     }
-    return linear_enqueue(slab, parts, dW, dX, dBias, dY, M, N, K, s, static_cast<char*>(sc->p));
+    return linear_enqueue(p, dW, dX, dBias, dY, M, N, K, s, static_cast<char*>(sc->p));
 }
 
 int vvli_gpu_linear_noalloc(const uint16_t* dW, const float* dX, const uint16_t* dBias, float* dY, uint32_t M,
                             uint32_t N, uint32_t K, void* stream) {
     int rc = check_linear_args(dW, dX, dY, M, N, K, "vvli_gpu_linear_noalloc");
     if (rc) return rc;
-    const bool slab = linear_uses_slab(dW, dX, M, N, K);
-    const size_t payload = linear_payload_bytes(slab, M, N, K);
-    // (The bound that callers know is that of the split planes, M > 64.)
-    const size_t bound = std::max(payload, linear_payload_bytes(false, M, N, K));
+    // (The bound that callers know is that of the lean plan: M > 64 its planes.)
+    LinearPlan p = linear_plan(dW, dX, M, N, K);
+    const LinearPlan lean = linear_plan(dW, dX, M, N, K, true);
+    const size_t bound = std::max(p.payload, lean.payload);
     if (bound > kNoAllocScratchBytes)
         return set_error(VVLI_INVALID_CONFIG,
                          "vvli_gpu_linear_noalloc: M=%u N=%u K=%u needs %zu bytes of scratch, more than its %zu", M, N,
                          K, bound, kNoAllocScratchBytes);
-    const size_t part_bytes = slab ? 0 : linear_part_bytes(M, N, K);
-    const bool parts = part_bytes > 0 && part_bytes <= kNoAllocPartBytes;
+    if (p.part > kNoAllocPartBytes) p = lean;
     char* mem = nullptr;
-    if (payload && (rc = scratch_on_device(&mem))) return rc;
-    return linear_enqueue(slab, parts, dW, dX, dBias, dY, M, N, K, static_cast<hipStream_t>(stream), mem);
+    if (p.bytes() && (rc = scratch_on_device(&mem))) return rc;
+    return linear_enqueue(p, dW, dX, dBias, dY, M, N, K, static_cast<hipStream_t>(stream), mem);
+}
+
+int vvli_gpu_test_linear_route(uint32_t M, uint32_t N, uint32_t K, uint32_t cus, vvli_gpu_linear_route* out) {
+    if (!out) return set_error(VVLI_NULL_ARG, "NULL argument to vvli_gpu_test_linear_route");
+    if (M == 0 || N == 0 || K == 0 || K % 8 != 0 || cus == 0)
+        return set_error(VVLI_INVALID_CONFIG, "bad linear route M=%u N=%u K=%u cus=%u", M, N, K, cus);
+    const LinearPlan p = linear_plan(M, N, K, true, false, cus);
+    out->kernel = static_cast<uint32_t>(p.kernel);
+    out->splits = p.splits;
+    out->gemm_few_rows = gemm_plain_plan(M, N, K, cus).few_rows;
+    out->scratch_bytes = p.bytes();
+    return VVLI_OK;
 }
 
 }  // extern "C"

@@ -1249,7 +1249,7 @@ __global__ __launch_bounds__(256) void zero_rows_kernel(float* __restrict__ out,
 // output rows are dense (they are zeroed first); SwiGLU tiles only with a
 // gate/up scratch (the epilogue is nonlinear: the sums go there and a
 // separate pass applies it).
-static uint32_t gemm_cus() {
+uint32_t gemm_cus() {
     static const uint32_t cus = [] {
         int dev = 0, n = 0;
         if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) !=
@@ -1260,9 +1260,9 @@ static uint32_t gemm_cus() {
     return cus;
 }
 
-uint32_t gemm_k_splits(int mode, const GemmArgs& g, uint32_t tiles) {
+// What follows plans a launch on a device of `cus` CUs.
+static uint32_t gemm_k_splits(int mode, const GemmArgs& g, uint32_t tiles, uint32_t cus) {
     if ((mode == kGemmGateUp && !g.gu_acc) || (mode == kGemmPlain && g.ldo != g.N)) return 1;
-    const uint32_t cus = gemm_cus();
     const uint32_t nk = (g.K + kBK - 1) / kBK;
     // Each split keeps at least 8 K steps (16 once there are 32 tiles: then
     // half the CUs with twice the steps beat a full round of short loops,
@@ -1276,7 +1276,8 @@ uint32_t gemm_k_splits(int mode, const GemmArgs& g, uint32_t tiles) {
     return splits;
 }
 
-size_t gemm_part_elems() { return static_cast<size_t>(gemm_cus()) * kBM * kBN; }
+static size_t gemm_part_elems(uint32_t cus) { return static_cast<size_t>(cus) * kBM * kBN; }
+size_t gemm_part_elems() { return gemm_part_elems(gemm_cus()); }
 
 // What a launch costs on each tile, in us: a round over the CUs takes 7 to 7.5
 // us and, per K step of 32, 0.90 on 128 x 256, 1.48 on 256 x 256, 0.47 on
@@ -1287,8 +1288,8 @@ size_t gemm_part_elems() { return static_cast<size_t>(gemm_cus()) * kBM * kBN; }
 // 60 / 47 / 70; 2048 x 4096 x 2048 80 / 100 / 87; 512 x 8192 x 2048 55 / 97 /
 // 46; 512 x 18000 x 1000 83 / 63 / 78; 200 x 2048 x 8192 50 / 320 / 35;
 // 130 x 1000 x 4000 29 / 159 / 26.
-static float gemm_tile_us(int mode, const GemmArgs& g, uint32_t cols, uint32_t splits) {
-    const uint32_t cus = gemm_cus(), nk = (g.K + kBK - 1) / kBK;
+static float gemm_tile_us(int mode, const GemmArgs& g, uint32_t cols, uint32_t splits, uint32_t cus) {
+    const uint32_t nk = (g.K + kBK - 1) / kBK;
     const uint32_t tiles = ((cols + kBN - 1) / kBN) * ((g.M + kBM - 1) / kBM);
     const float mb = 4e-6f * splits * g.M * cols;
     float us = ((tiles * splits + cus - 1) / cus) * (7.5f + 0.9f * ((nk + splits - 1) / splits));
@@ -1296,19 +1297,19 @@ static float gemm_tile_us(int mode, const GemmArgs& g, uint32_t cols, uint32_t s
     if (splits > 1 && mode == kGemmGateUp) us += 5.f;  // the SwiGLU pass
     return us;
 }
-static float gemm_wide_us(const GemmArgs& g, uint32_t cols) {
-    const uint32_t cus = gemm_cus(), tiles = ((cols + kWN - 1) / kWN) * ((g.M + kWM - 1) / kWM);
+static float gemm_wide_us(const GemmArgs& g, uint32_t cols, uint32_t cus) {
+    const uint32_t tiles = ((cols + kWN - 1) / kWN) * ((g.M + kWM - 1) / kWM);
     return ((tiles + cus - 1) / cus) * (7.f + 1.48f * ((g.K + kBK - 1) / kBK));
 }
 // (splits: the best for the tile, at least four stages of K each)
-static float gemm_square_us(int mode, const GemmArgs& g, uint32_t cols, uint32_t& splits) {
-    const uint32_t cus = gemm_cus(), tiles = ((cols + kSqN - 1) / kSqN) * ((g.M + kSqM - 1) / kSqM);
+static float gemm_square_us(int mode, const GemmArgs& g, uint32_t cols, uint32_t cus, uint32_t& splits) {
+    const uint32_t tiles = ((cols + kSqN - 1) / kSqN) * ((g.M + kSqM - 1) / kSqM);
     const uint32_t nk = (g.K + kSqK - 1) / kSqK;
     const uint32_t most = mode != kGemmGateUp && g.part ? std::max(1u, std::min(kMaxPartSplits, nk / 4)) : 1u;
     float best = 0.f;
     for (uint32_t want = 1; want <= most; ++want) {
         const uint32_t per = (nk + want - 1) / want, sp = (nk + per - 1) / per;  // every split gets K steps
-        if (sp > 1 && static_cast<size_t>(sp) * g.M * g.N > gemm_part_elems()) break;
+        if (sp > 1 && static_cast<size_t>(sp) * g.M * g.N > gemm_part_elems(cus)) break;
         float us = ((tiles * sp + cus - 1) / cus) * (7.f + 0.94f * per);
         if (sp > 1) us += (mode == kGemmResid ? 0.5f : 3.f) + 4e-6f * sp * g.M * g.N / 2.5f;
         if (want == 1 || us < best) best = us, splits = sp;
@@ -1343,14 +1344,14 @@ struct GemmPlan {
 
 // Splits of the few-row kernel: enough items for a block per CU, the fewest
 // splits with the same longest K range, at most kMaxPartSplits.
-static uint32_t slab_splits(uint32_t tiles, uint32_t K, uint32_t M) {
+static uint32_t slab_splits(uint32_t tiles, uint32_t K, uint32_t M, uint32_t cus) {
     const uint32_t kc = M > 64 ? 64 : 128, nch = (K + kc - 1) / kc;
-    const uint32_t most = std::max(1u, std::min({gemm_cus() / tiles, kMaxPartSplits, nch}));
+    const uint32_t most = std::max(1u, std::min({cus / tiles, kMaxPartSplits, nch}));
     const uint32_t per = (nch + most - 1) / most;
     return (nch + per - 1) / per;
 }
 
-static GemmPlan gemm_plan(int mode, const GemmArgs& g) {
+static GemmPlan gemm_plan(int mode, const GemmArgs& g, uint32_t cus) {
     const uint32_t cols = mode == kGemmGateUp ? 2 * g.N : g.N;
     // Few rows: the slab kernel. Up to 64 rows always (one layer of the 1B
     // shape at 45 rows: gate/up 36 -> 20 us with its zeroing and SwiGLU passes,
@@ -1359,30 +1360,27 @@ static GemmPlan gemm_plan(int mode, const GemmArgs& g) {
     // tiles, 18944 x 3584 102 against 61).
     if (g.M <= kSlabMaxRows && (mode != kGemmPlain || g.ldo == g.N || !g.part)) {
         const uint32_t tiles = (cols + kSlabN - 1) / kSlabN;
-        const uint32_t splits = mode != kGemmGateUp && g.part ? slab_splits(tiles, g.K, g.M) : 1u;
-        if (g.M <= 64 || tiles * splits <= gemm_cus()) return {GemmKernel::Slab, splits};
+        const uint32_t splits = mode != kGemmGateUp && g.part ? slab_splits(tiles, g.K, g.M, cus) : 1u;
+        if (g.M <= 64 || tiles * splits <= cus) return {GemmKernel::Slab, splits};
     }
     const uint32_t gx = (cols + kBN - 1) / kBN, gy = (g.M + kBM - 1) / kBM;
-    const uint32_t splits = gemm_k_splits(mode, g, gx * gy);
+    const uint32_t splits = gemm_k_splits(mode, g, gx * gy, cus);
     uint32_t sq_splits = 1;
-    const float tile = gemm_tile_us(mode, g, cols, splits), wide = gemm_wide_us(g, cols);
-    const float square = gemm_square_us(mode, g, cols, sq_splits);
+    const float tile = gemm_tile_us(mode, g, cols, splits, cus), wide = gemm_wide_us(g, cols, cus);
+    const float square = gemm_square_us(mode, g, cols, cus, sq_splits);
     if (square < tile && square < wide) return {GemmKernel::Square, sq_splits};
     if (wide < tile) return {GemmKernel::Wide, 1};
     return {GemmKernel::Tile, splits};
 }
 
-uint32_t gemm_splits(int mode, const GemmArgs& g) { return gemm_plan(mode, g).splits; }
+uint32_t gemm_splits(int mode, const GemmArgs& g) { return gemm_plan(mode, g, gemm_cus()).splits; }
 
-uint32_t gemm_plain_part_splits(uint32_t M, uint32_t N, uint32_t K) {
+PlainGemmPlan gemm_plain_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t cus) {
     static float there;  // only that `part` is given counts
     GemmArgs g;
     g.M = M, g.N = N, g.K = K, g.ldo = N, g.part = &there;
-    return gemm_plan(kGemmPlain, g).splits;
-}
-
-uint32_t gemm_slab_part_splits(uint32_t M, uint32_t N, uint32_t K) {
-    return M <= kSlabMaxRows ? slab_splits((N + kSlabN - 1) / kSlabN, K, M) : 1;
+    const GemmPlan p = gemm_plan(kGemmPlain, g, cus);
+    return {p.kernel == GemmKernel::Slab, p.splits};
 }
 
 template <int MODE, int MT, int KC, int ST, int WM, int WN, bool F32A>
@@ -1428,16 +1426,13 @@ size_t gemm_split_elems(uint32_t M, uint32_t K) { return static_cast<size_t>(2) 
 
 hipError_t launch_gemm_bf16(int mode, const GemmArgs& g, hipStream_t s) {
     if (g.M == 0 || g.N == 0) return hipSuccess;
-    const GemmPlan plan = gemm_plan(mode, g);
-    // The few-row kernel splits f32 rows itself.
-    const bool f32a = plan.kernel == GemmKernel::Slab && mode == kGemmPlain && !g.a_ready && !g.norm_w && !g.a_rows &&
-                      g.a && g.lda % 4 == 0 && reinterpret_cast<uintptr_t>(g.a) % 16 == 0;
-    if ((!g.a_hl && !f32a) || g.K % 8 != 0 || (g.norm_w && !g.row_scale)) return hipErrorInvalidValue;
+    const GemmPlan plan = gemm_plan(mode, g, gemm_cus());
+    if (!g.a_hl || g.K % 8 != 0 || (g.norm_w && !g.row_scale)) return hipErrorInvalidValue;
     if ((g.out_hl && mode != kGemmGateUp) || (!g.out_hl && !g.out) ||
         (g.a_plane && g.a_plane < static_cast<size_t>(g.M) * gemm_kp(g.K)) ||
         (g.out_hl && g.out_plane < static_cast<size_t>(g.M) * gemm_kp(g.N)))
         return hipErrorInvalidValue;
-    if (!g.a_ready && !f32a) {
+    if (!g.a_ready) {
         const size_t n = static_cast<size_t>(g.M) * (gemm_kp(g.K) / 8);
         hipError_t e = vlaunch(gemm_split_kernel, dim3(static_cast<uint32_t>((n + 255) / 256)), dim3(256), 0, s, g);
         if (e != hipSuccess) return e;
@@ -1446,7 +1441,7 @@ hipError_t launch_gemm_bf16(int mode, const GemmArgs& g, hipStream_t s) {
         if (plan.splits > 1 && static_cast<size_t>(plan.splits) * g.M * g.N > gemm_part_elems()) return hipErrorInvalidValue;
         if (mode == kGemmGateUp) return launch_slab<kGemmGateUp, false>(g, plan.splits, s);
         if (mode == kGemmResid) return launch_slab<kGemmResid, false>(g, plan.splits, s);
-        return f32a ? launch_slab<kGemmPlain, true>(g, plan.splits, s) : launch_slab<kGemmPlain, false>(g, plan.splits, s);
+        return launch_slab<kGemmPlain, false>(g, plan.splits, s);
     }
     static const hipError_t attr = [] {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_bf16_kernel<kGemmPlain>),
@@ -1495,6 +1490,17 @@ hipError_t launch_gemm_bf16(int mode, const GemmArgs& g, hipStream_t s) {
         case kGemmGateUp: return vlaunch(gemm_bf16_kernel<kGemmGateUp>, grid, dim3(kGemmThreads), kGemmLds, s, g);
         default: return hipErrorInvalidValue;
     }
+}
+
+hipError_t launch_gemm_few_rows(const GemmArgs& g, uint32_t splits, hipStream_t s) {
+    if (g.M == 0 || g.N == 0) return hipSuccess;
+    const uint32_t nch = (g.K + (g.M > 64 ? 63 : 127)) / (g.M > 64 ? 64 : 128);
+    const auto aligned = [](const void* p) { return p && reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+    if (g.M > kSlabMaxRows || g.K % 8 != 0 || g.lda % 4 != 0 || !aligned(g.a) || !aligned(g.w[0]) || !g.out ||
+        g.seg_end[0] != g.N || splits == 0 || splits > nch || (nch + splits - 1) / splits * (splits - 1) >= nch ||
+        (splits > 1 && (!g.part || static_cast<size_t>(splits) * g.M * g.N > gemm_part_elems())))
+        return hipErrorInvalidValue;
+    return launch_slab<kGemmPlain, true>(g, splits, s);
 }
 
 hipError_t launch_slab_reduce(const float* part, float* out, size_t n, uint32_t splits, hipStream_t s) {

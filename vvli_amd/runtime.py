@@ -411,6 +411,16 @@ def linear(dW: int, dX: int, dY: int, M: int, N: int, K: int, dBias: int | None 
                                           c_void_p(dY), M, N, K, None if stream is None else c_void_p(stream)))
 
 
+LINEAR_KERNELS = ("gemv", "skinny", "few_rows", "tiles")
+
+
+def linear_route(M: int, N: int, K: int, cus: int = 256) -> _lib.CLinearRoute:
+    """vvli_gpu_test_linear_route: what ``linear`` runs on a device of ``cus`` compute units (no GPU needed)."""
+    out = _lib.CLinearRoute()
+    _lib.check(_lib.lib().vvli_gpu_test_linear_route(M, N, K, cus, byref(out)))
+    return out
+
+
 def linear_noalloc(dW: int, dX: int, dY: int, M: int, N: int, K: int, dBias: int | None = None,
                    stream: int | None = None) -> None:
     """vvli_gpu_linear_noalloc: the same op with its scratch in a static device
