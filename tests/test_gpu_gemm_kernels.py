@@ -76,27 +76,109 @@ def test_few_rows_unaligned_and_repeated():
     assert torch.equal(y, y2)  # the splits are added in a fixed order
 
 
-def test_few_rows_under_capture():
-    """A call that needed no scratch before its first use can still be captured
-    on a fresh stream, and replays give the eager result."""
+def linear_call(w, x, y, stream):
+    R.linear(w.data_ptr(), x.data_ptr(), y.data_ptr(), x.shape[0], w.shape[0], w.shape[1], None, stream.cuda_stream)
+
+
+def replays(graph, y, e, exact, between):
+    """Three replays, eager work and a synchronization between them, each against the eager result."""
     import torch
 
-    M, N, K = 16, 2048, 2048
+    for _ in range(3):
+        y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        if exact:
+            assert torch.equal(y, e)
+        else:
+            assert float((y - e).norm() / e.norm()) <= 1e-5  # sum orders of the same 16-bit products
+        between()
+
+
+def test_few_rows_under_capture():
+    """A call that the few-row GEMM runs with scratch and the skinny kernel
+    without takes the latter under capture: on a fresh stream, and with no
+    address of the stream's scratch in the graph."""
+    import torch
+
+    M, N, K = 33, 2048, 2048
+    eager, cap = R.linear_route(M, N, K), R.linear_route(M, N, K, captured=True)
+    assert R.LINEAR_KERNELS[eager.kernel] == "few_rows" and eager.scratch_bytes > 0
+    assert R.LINEAR_KERNELS[cap.kernel] == "skinny" and cap.scratch_bytes == 0
     w = (torch.randn(N, K, device="cuda") * 0.02).bfloat16()
     x = torch.randn(M, K, device="cuda")
     y, e = torch.empty(M, N, device="cuda"), torch.empty(M, N, device="cuda")
-    R.linear(w.data_ptr(), x.data_ptr(), e.data_ptr(), M, N, K, None, torch.cuda.current_stream().cuda_stream)
+    linear_call(w, x, e, torch.cuda.current_stream())
     st = torch.cuda.Stream()
     st.wait_stream(torch.cuda.current_stream())
     g = torch.cuda.CUDAGraph()
     with torch.cuda.graph(g, stream=st):
-        R.linear(w.data_ptr(), x.data_ptr(), y.data_ptr(), M, N, K, None, torch.cuda.current_stream().cuda_stream)
-    for _ in range(3):
-        y.zero_()
-        g.replay()
-        torch.cuda.synchronize()
-        assert float((y - e).norm() / e.norm()) <= 1e-5  # sum orders of the same 16-bit products
-        x += 0  # eager work between the replays
+        linear_call(w, x, y, torch.cuda.current_stream())
+    replays(g, y, e, False, lambda: x.add_(0))
+
+
+# Calls that keep scratch under capture: K-split partials of the few-row GEMM
+# and of the skinny kernel, split planes with partials and without.
+CAPTURED = [(16, 2048, 8192), (5, 16, 8192), (512, 2048, 2048), (300, 9000, 512)]
+
+
+@pytest.mark.parametrize("M,N,K", CAPTURED)
+def test_captured_scratch_outlives_growth(M, N, K):
+    """The usual order: a warm-up call, the capture, then larger eager calls on
+    that stream, which free and replace the scratch of its eager calls, and the
+    replays on another stream beside them."""
+    import torch
+
+    assert R.linear_route(M, N, K, captured=True).scratch_bytes > 0
+    w = (torch.randn(N, K, device="cuda") * 0.02).bfloat16()
+    x = torch.randn(M, K, device="cuda")
+    y, e = torch.empty(M, N, device="cuda"), torch.empty(M, N, device="cuda")
+    wl = (torch.randn(256, 8192, device="cuda") * 0.02).bfloat16()
+    xl = torch.randn(1500, 8192, device="cuda")
+    yl = torch.empty(1500, 256, device="cuda")
+    ref = xl[:2].double() @ wl.double().t()
+    st = torch.cuda.Stream()
+    st.wait_stream(torch.cuda.current_stream())
+    linear_call(w, x, e, st)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=st):
+        linear_call(w, x, y, torch.cuda.current_stream())
+    rows = [500]
+
+    def larger():  # one row more each time: its scratch grows again
+        linear_call(wl, xl[: rows[0]], yl[: rows[0]], st)
+        rows[0] += 500
+        st.synchronize()
+        assert float((yl[:2].double() - ref).norm() / ref.norm()) <= 1e-4
+
+    larger()
+    replays(g, y, e, True, larger)
+
+
+@pytest.mark.parametrize("M,N,K", CAPTURED)
+def test_first_call_of_a_stream_under_capture(M, N, K):
+    """The capture's scratch is not the stream's: an eager call before the
+    first replay, and one after the graph is gone, have their own."""
+    import torch
+
+    w = (torch.randn(N, K, device="cuda") * 0.02).bfloat16()
+    x = torch.randn(M, K, device="cuda")
+    y, y2, e = (torch.zeros(M, N, device="cuda") for _ in range(3))
+    linear_call(w, x, e, torch.cuda.current_stream())
+    st = torch.cuda.Stream()
+    st.wait_stream(torch.cuda.current_stream())
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=st):
+        linear_call(w, x, y, torch.cuda.current_stream())
+    linear_call(w, x, y2, st)
+    torch.cuda.synchronize()
+    assert torch.equal(y2, e) and not bool(y.any())
+    replays(g, y, e, True, lambda: linear_call(w, x, y2, st))
+    del g
+    y2.zero_()
+    linear_call(w, x, y2, st)
+    torch.cuda.synchronize()
+    assert torch.equal(y2, e)
 
 
 def rel_err(got, ref):
@@ -165,8 +247,8 @@ def test_square_tile_prefill():
 
 
 def test_square_tile_under_capture():
-    """A K-split call captured with scratch for its split planes alone (a
-    smaller call came before it on that stream) takes no more of it."""
+    """A K-split call captured after a smaller one on that stream, whose scratch
+    would not hold its partial sums."""
     import torch
 
     K = 2048

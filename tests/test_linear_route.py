@@ -34,3 +34,25 @@ def test_few_rows_past_one_round_of_a_small_device():
     assert kernel(R.linear_route(128, 16384, 2048, 256)) == "few_rows"
     assert kernel(R.linear_route(128, 16384, 2048, 128)) == "tiles"
     assert kernel(R.linear_route(100, 4096, 2048, 32)) == "tiles"
+
+
+def test_captured_calls_that_can_do_without_scratch_do():
+    """Up to 64 rows a captured call either runs a kernel without scratch, or
+    one that needs it eager too; larger ones run as eager ones do."""
+    seen = 0
+    for M in ROWS:
+        for N, K in SIZES + [(2048, 4096), (3584, 3584), (512, 4096), (1152, 896)]:
+            e, c = R.linear_route(M, N, K), R.linear_route(M, N, K, captured=True)
+            if M > 64 or e.scratch_bytes == 0:
+                assert c.scratch_bytes == e.scratch_bytes, (M, N, K)
+            if M > 64:
+                assert (c.kernel, c.splits) == (e.kernel, e.splits), (M, N, K)
+            if c.scratch_bytes == 0 and e.scratch_bytes > 0:
+                assert kernel(e) == "few_rows" and kernel(c) == "skinny" and c.splits == 1
+                seen += 1
+    assert seen > 0
+    # 33 x 2048 x 2048: K splits of the few-row GEMM, or the unsplit skinny kernel
+    assert R.linear_route(33, 2048, 2048).scratch_bytes > 0
+    assert R.linear_route(33, 2048, 2048, captured=True).scratch_bytes == 0
+    # 16 x 2048 x 8192: the skinny kernel would split K too
+    assert R.linear_route(16, 2048, 8192, captured=True).scratch_bytes > 0

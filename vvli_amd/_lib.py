@@ -156,7 +156,7 @@ PROTOTYPES = {
     "vvli_gpu_linear": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_uint32, c_uint32, c_uint32, c_void_p]),
     "vvli_gpu_linear_noalloc": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_uint32, c_uint32, c_uint32,
                                         c_void_p]),
-    "vvli_gpu_test_linear_route": (c_int, [c_uint32, c_uint32, c_uint32, c_uint32, POINTER(CLinearRoute)]),
+    "vvli_gpu_test_linear_route": (c_int, [c_uint32, c_uint32, c_uint32, c_uint32, c_uint32, POINTER(CLinearRoute)]),
     "vvli_host_fill_deterministic": (None, [c_void_p, c_size_t, c_uint32]),
     "vvli_host_fill_synthetic": (c_int, [POINTER(CConfig), c_uint64, c_float, c_void_p, c_size_t, c_uint32]),
     "vvli_host_synthetic_normal": (c_double, [c_uint64, c_uint64, c_uint64]),

@@ -3,9 +3,10 @@
 // Y[m,n] = sum_k bf16 W[n,k] * X[m,k] (+ bias[n]), f32 accumulation.
 //
 // Two entry points share one enqueue routine and therefore the same kernels
-// and results; they differ only in where the GEMM's activation split planes
-// live: vvli_gpu_linear keeps a stream-ordered allocation per stream,
-// vvli_gpu_linear_noalloc uses a static device array and allocates nothing.
+// and results; they differ only in where a call's scratch lives:
+// vvli_gpu_linear keeps a stream-ordered allocation per stream (and a block of
+// its own for calls under capture), vvli_gpu_linear_noalloc uses a static
+// device array and allocates nothing.
 #include <algorithm>
 #include <mutex>
 #include <utility>
@@ -449,6 +450,10 @@ LinearPlan linear_plan(const uint16_t* dW, const float* dX, uint32_t M, uint32_t
     return linear_plan(M, N, K, aligned, lean, gemm_cus());
 }
 
+// Under capture a call that can do without scratch does, so that its graph
+// stands alone; the others run as ever.
+LinearPlan captured_plan(const LinearPlan& plan, const LinearPlan& lean) { return lean.bytes() == 0 ? lean : plan; }
+
 // Enqueue the op on s. scratch: p.bytes() of device memory laid out as above
 // (null when that is 0).
 int linear_enqueue(const LinearPlan& p, const uint16_t* dW, const float* dX, const uint16_t* dBias, float* dY, uint32_t M,
@@ -489,6 +494,23 @@ int linear_enqueue(const LinearPlan& p, const uint16_t* dW, const float* dX, con
     return VVLI_OK;
 }
 
+// Scratch for calls under capture: allocated and its counters cleared on a
+// stream of its own, complete on return, so that the capture records neither.
+hipError_t alloc_outside_capture(void** out, size_t bytes) {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;  // this thread may allocate during a capture
+    hipError_t e = hipThreadExchangeStreamCaptureMode(&mode);
+    if (e != hipSuccess) return e;
+    hipStream_t s = nullptr;
+    e = hipMalloc(out, bytes);
+    if (e == hipSuccess) e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
+    if (e == hipSuccess) e = hipMemsetAsync(*out, 0, kCounterBytes, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (s) (void)hipStreamDestroy(s);
+    if (e != hipSuccess && *out) (void)hipFree(*out);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return e;
+}
+
 // Device address of `scratch` on the current device, looked up on the
 // device's first call (hipGetSymbolAddress with that device current) and
 // kept per device: every GPU holds its own copy at its own address.
@@ -522,13 +544,25 @@ int vvli_gpu_linear(const uint16_t* dW, const float* dX, const uint16_t* dBias, 
     hipStream_t s = static_cast<hipStream_t>(stream);
     LinearPlan p = linear_plan(dW, dX, M, N, K);
     if (p.bytes() == 0) return linear_enqueue(p, dW, dX, dBias, dY, M, N, K, s, nullptr);
-    // The scratch is kept per stream and grows stream-ordered (its counters
-    // cleared once per allocation); the lock covers the enqueue, so calls on
-    // one stream use it in turn.
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) != hipSuccess) (void)hipGetLastError();  // (the launch reports it)
+    const bool captured = cap != hipStreamCaptureStatusNone;
+    if (captured) {
+        p = captured_plan(p, linear_plan(dW, dX, M, N, K, true));
+        if (p.bytes() == 0) return linear_enqueue(p, dW, dX, dBias, dY, M, N, K, s, nullptr);
+    }
+    // Scratch is kept per stream; the lock covers the enqueue, so calls on one
+    // stream use it in turn. Eager calls grow theirs stream-ordered (its
+    // counters cleared once per allocation). A graph outlives the call that it
+    // records, may be replayed on any stream and is not seen again here: calls
+    // under capture have a block of their own, never freed, so that no growth
+    // and no eager call touches what a replay uses.
     struct StreamScratch {
         hipStream_t stream;
         void* p;
         size_t bytes;
+        void* captured;
+        size_t captured_bytes;
     };
     static std::mutex mu;
     static std::vector<StreamScratch> cache;
@@ -537,18 +571,19 @@ int vvli_gpu_linear(const uint16_t* dW, const float* dX, const uint16_t* dBias, 
     for (StreamScratch& c : cache)
         if (c.stream == s) sc = &c;
     if (!sc) {
-        cache.push_back(StreamScratch{s, nullptr, 0});
+        cache.push_back(StreamScratch{s, nullptr, 0, nullptr, 0});
         sc = &cache.back();
     }
-    if (sc->bytes < p.bytes() && (p.kernel == LinearKernel::FewRows || p.part > 0)) {
-        // Under stream capture nothing may be allocated for a call that the
-        // other kernels serve without scratch or with less: they take it.
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
-            (void)hipGetLastError();
-            p = linear_plan(dW, dX, M, N, K, true);
-            if (p.bytes() == 0) return linear_enqueue(p, dW, dX, dBias, dY, M, N, K, s, nullptr);
+    if (captured) {
+        if (sc->captured_bytes < p.bytes()) {
+            // (sizes double, so that all blocks of a stream are less than two of its largest)
+            size_t bytes = 1u << 20;
+            while (bytes < p.bytes()) bytes *= 2;
+            void* block = nullptr;
+            HIP_TRY(alloc_outside_capture(&block, bytes));
+            sc->captured = block, sc->captured_bytes = bytes;
         }
+        return linear_enqueue(p, dW, dX, dBias, dY, M, N, K, s, static_cast<char*>(sc->captured));
     }
     if (sc->bytes < p.bytes()) {
         if (sc->p) HIP_TRY(hipFreeAsync(sc->p, s));
@@ -578,11 +613,13 @@ int vvli_gpu_linear_noalloc(const uint16_t* dW, const float* dX, const uint16_t*
     return linear_enqueue(p, dW, dX, dBias, dY, M, N, K, static_cast<hipStream_t>(stream), mem);
 }
 
-int vvli_gpu_test_linear_route(uint32_t M, uint32_t N, uint32_t K, uint32_t cus, vvli_gpu_linear_route* out) {
+int vvli_gpu_test_linear_route(uint32_t M, uint32_t N, uint32_t K, uint32_t cus, uint32_t captured,
+                               vvli_gpu_linear_route* out) {
     if (!out) return set_error(VVLI_NULL_ARG, "NULL argument to vvli_gpu_test_linear_route");
     if (M == 0 || N == 0 || K == 0 || K % 8 != 0 || cus == 0)
         return set_error(VVLI_INVALID_CONFIG, "bad linear route M=%u N=%u K=%u cus=%u", M, N, K, cus);
-    const LinearPlan p = linear_plan(M, N, K, true, false, cus);
+    LinearPlan p = linear_plan(M, N, K, true, false, cus);
+    if (captured) p = captured_plan(p, linear_plan(M, N, K, true, true, cus));
     out->kernel = static_cast<uint32_t>(p.kernel);
     out->splits = p.splits;
     out->gemm_few_rows = gemm_plain_plan(M, N, K, cus).few_rows;
