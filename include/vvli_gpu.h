@@ -340,9 +340,9 @@ int vvli_gpu_test_sampler_trace(const float* logits, uint32_t n, const vvli_gpu_
  * GEMM path where K is split more than eight ways: they are then added with
  * atomics (the last bits may vary run to run). Scratch (K-split partials and
  * counters, or the GEMM's planes, about 4*M*K bytes, and its K-split partials,
- * at most 32 MiB) is kept per stream: allocated stream-ordered, and freed and
- * allocated anew when a later call on that stream needs more (calls on one
- * stream use it in turn). Under stream capture a call with M <= 64 that can
+ * at most 32 MiB; without the partials where there is no memory for them) is
+ * kept per stream: allocated stream-ordered, and freed and allocated anew when
+ * a later call on that stream needs more (calls on one stream use it in turn). Under stream capture a call with M <= 64 that can
  * run without scratch does; any other records the addresses of a second block
  * of that stream, which no eager call uses, and which is allocated outside the
  * capture and kept until the process ends, as are the smaller blocks that it
@@ -369,15 +369,18 @@ int vvli_gpu_linear_noalloc(const uint16_t* dW, const float* dX, const uint16_t*
                             uint32_t N, uint32_t K, void* stream);
 
 /* Test hook of vvli_gpu_linear (no reference counterpart; needs no GPU): what
- * a call with 16-byte aligned dW and dX, eager or captured, runs on a device
- * of `cus` compute units. kernel: 0 GEMV, 1 skinny, 2 few-row GEMM, 3 tiles; splits: of K;
+ * a call with 16-byte aligned dW and dX runs on a device of `cus` compute
+ * units (flags: captured; lean, when there is no memory for partial sums).
+ * kernel: 0 GEMV, 1 skinny, 2 few-row GEMM, 3 tiles; splits: of K;
  * gemm_few_rows: whether the prefill GEMM, given these sizes, would run its
  * few-row kernel; scratch_bytes: scratch of the call (0: none). */
+#define VVLI_ROUTE_CAPTURED 1u
+#define VVLI_ROUTE_LEAN 2u
 typedef struct vvli_gpu_linear_route {
     uint32_t kernel, splits, gemm_few_rows, reserved;
     uint64_t scratch_bytes;
 } vvli_gpu_linear_route;
-int vvli_gpu_test_linear_route(uint32_t M, uint32_t N, uint32_t K, uint32_t cus, uint32_t captured,
+int vvli_gpu_test_linear_route(uint32_t M, uint32_t N, uint32_t K, uint32_t cus, uint32_t flags,
                                vvli_gpu_linear_route* out);
 
 #ifdef __cplusplus

@@ -56,3 +56,18 @@ def test_captured_calls_that_can_do_without_scratch_do():
     assert R.linear_route(33, 2048, 2048, captured=True).scratch_bytes == 0
     # 16 x 2048 x 8192: the skinny kernel would split K too
     assert R.linear_route(16, 2048, 8192, captured=True).scratch_bytes > 0
+
+
+def test_without_memory_for_partial_sums():
+    """What runs when the scratch of a call cannot be had: no more than the
+    skinny kernel's own (M <= 64) or the split planes need."""
+    for M in ROWS:
+        for N, K in SIZES + [(2048, 4096), (3584, 3584), (512, 4096), (1152, 896)]:
+            e, l = R.linear_route(M, N, K), R.linear_route(M, N, K, lean=True)
+            assert kernel(l) != "few_rows"
+            if M > 64:
+                assert kernel(l) == "tiles" and l.scratch_bytes == 64 * 1024 + 4 * M * (-(-K // 32) * 32)
+            elif kernel(l) == "skinny" and l.splits == 1 or kernel(l) == "gemv":
+                assert l.scratch_bytes == 0
+            if kernel(e) == kernel(l):
+                assert l.scratch_bytes <= e.scratch_bytes

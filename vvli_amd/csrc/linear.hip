@@ -574,25 +574,41 @@ int vvli_gpu_linear(const uint16_t* dW, const float* dX, const uint16_t* dBias, 
         cache.push_back(StreamScratch{s, nullptr, 0, nullptr, 0});
         sc = &cache.back();
     }
+    // Memory for p, or for the lean plan where there is no more: what the
+    // partial sums of a K split need beyond it must not fail a call.
+    auto fit = [&](size_t have, auto&& alloc) {
+        if (have >= p.bytes()) return hipSuccess;
+        hipError_t e = alloc(p.bytes());
+        const LinearPlan lean = linear_plan(dW, dX, M, N, K, true);
+        if (e != hipErrorOutOfMemory || lean.bytes() >= p.bytes()) return e;
+        (void)hipGetLastError();
+        p = lean;
+        return p.bytes() ? alloc(p.bytes()) : hipSuccess;
+    };
+    char* mem = nullptr;
     if (captured) {
-        if (sc->captured_bytes < p.bytes()) {
+        HIP_TRY(fit(sc->captured_bytes, [&](size_t need) {
             // (sizes double, so that all blocks of a stream are less than two of its largest)
             size_t bytes = 1u << 20;
-            while (bytes < p.bytes()) bytes *= 2;
+            while (bytes < need) bytes *= 2;
             void* block = nullptr;
-            HIP_TRY(alloc_outside_capture(&block, bytes));
-            sc->captured = block, sc->captured_bytes = bytes;
-        }
-        return linear_enqueue(p, dW, dX, dBias, dY, M, N, K, s, static_cast<char*>(sc->captured));
+            const hipError_t e = alloc_outside_capture(&block, bytes);
+            if (e == hipSuccess) sc->captured = block, sc->captured_bytes = bytes;
+            return e;
+        }));
+        mem = static_cast<char*>(sc->captured);
+    } else {
+        HIP_TRY(fit(sc->bytes, [&](size_t need) {
+            hipError_t e = sc->p ? hipFreeAsync(sc->p, s) : hipSuccess;
+            sc->p = nullptr, sc->bytes = 0;
+            if (e == hipSuccess) e = hipMallocAsync(&sc->p, need, s);
+            if (e == hipSuccess) e = hipMemsetAsync(sc->p, 0, kCounterBytes, s);
+            if (e == hipSuccess) sc->bytes = need;
+            return e;
+        }));
+        mem = static_cast<char*>(sc->p);
     }
-    if (sc->bytes < p.bytes()) {
-        if (sc->p) HIP_TRY(hipFreeAsync(sc->p, s));
-        sc->p = nullptr, sc->bytes = 0;
-        HIP_TRY(hipMallocAsync(&sc->p, p.bytes(), s));
-        HIP_TRY(hipMemsetAsync(sc->p, 0, kCounterBytes, s));
-        sc->bytes = p.bytes();
-    }
-    return linear_enqueue(p, dW, dX, dBias, dY, M, N, K, s, static_cast<char*>(sc->p));
+    return linear_enqueue(p, dW, dX, dBias, dY, M, N, K, s, p.bytes() ? mem : nullptr);
 }
 
 int vvli_gpu_linear_noalloc(const uint16_t* dW, const float* dX, const uint16_t* dBias, float* dY, uint32_t M,
@@ -613,13 +629,13 @@ int vvli_gpu_linear_noalloc(const uint16_t* dW, const float* dX, const uint16_t*
     return linear_enqueue(p, dW, dX, dBias, dY, M, N, K, static_cast<hipStream_t>(stream), mem);
 }
 
-int vvli_gpu_test_linear_route(uint32_t M, uint32_t N, uint32_t K, uint32_t cus, uint32_t captured,
+int vvli_gpu_test_linear_route(uint32_t M, uint32_t N, uint32_t K, uint32_t cus, uint32_t flags,
                                vvli_gpu_linear_route* out) {
     if (!out) return set_error(VVLI_NULL_ARG, "NULL argument to vvli_gpu_test_linear_route");
-    if (M == 0 || N == 0 || K == 0 || K % 8 != 0 || cus == 0)
+    if (M == 0 || N == 0 || K == 0 || K % 8 != 0 || cus == 0 || flags > (VVLI_ROUTE_CAPTURED | VVLI_ROUTE_LEAN))
         return set_error(VVLI_INVALID_CONFIG, "bad linear route M=%u N=%u K=%u cus=%u", M, N, K, cus);
-    LinearPlan p = linear_plan(M, N, K, true, false, cus);
-    if (captured) p = captured_plan(p, linear_plan(M, N, K, true, true, cus));
+    LinearPlan p = linear_plan(M, N, K, true, (flags & VVLI_ROUTE_LEAN) != 0, cus);
+    if (flags & VVLI_ROUTE_CAPTURED) p = captured_plan(p, linear_plan(M, N, K, true, true, cus));
     out->kernel = static_cast<uint32_t>(p.kernel);
     out->splits = p.splits;
     out->gemm_few_rows = gemm_plain_plan(M, N, K, cus).few_rows;
