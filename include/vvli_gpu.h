@@ -330,7 +330,8 @@ int vvli_gpu_test_sampler_trace(const float* logits, uint32_t n, const vvli_gpu_
  * pointers; K must be a multiple of 8; dY must be device memory (hipMalloc:
  * the K-split paths publish partials with write-through stores). stream:
  * hipStream_t or NULL for the null stream. Asynchronous: returns after the
- * launch. M <= 3 (and M = 4 when W has few row tiles) runs the
+ * launch. dW and dX need the alignment of their elements; from 64 rows on, dW at
+ * a 16-byte address is several times as fast. M <= 3 (and M = 4 when W has few row tiles) runs the
  * GEMV kernel, one launch for all rows of X (one per row when they do not fit
  * its LDS); otherwise 4 <= M <= 128 one kernel that reads W once and splits X
  * into two bf16 halves in registers, so that the products keep about 16 bits
@@ -369,13 +370,13 @@ int vvli_gpu_linear_noalloc(const uint16_t* dW, const float* dX, const uint16_t*
                             uint32_t N, uint32_t K, void* stream);
 
 /* Test hook of vvli_gpu_linear (no reference counterpart; needs no GPU): what
- * a call with 16-byte aligned dW and dX runs on a device of `cus` compute
- * units (flags: captured; lean, when there is no memory for partial sums).
- * kernel: 0 GEMV, 1 skinny, 2 few-row GEMM, 3 tiles; splits: of K;
+ * a call runs on a device of `cus` compute units (flags: captured; lean, when
+ * there is no memory for partial sums; dW not 16-byte aligned). kernel: 0 GEMV, 1 skinny, 2 few-row GEMM, 3 tiles; splits: of K;
  * gemm_few_rows: whether the prefill GEMM, given these sizes, would run its
  * few-row kernel; scratch_bytes: scratch of the call (0: none). */
 #define VVLI_ROUTE_CAPTURED 1u
 #define VVLI_ROUTE_LEAN 2u
+#define VVLI_ROUTE_UNALIGNED 4u
 typedef struct vvli_gpu_linear_route {
     uint32_t kernel, splits, gemm_few_rows, reserved;
     uint64_t scratch_bytes;

@@ -76,6 +76,24 @@ def test_few_rows_unaligned_and_repeated():
     assert torch.equal(y, y2)  # the splits are added in a fixed order
 
 
+@pytest.mark.parametrize("M,N,K", [(65, 200, 40), (100, 2048, 2048), (130, 300, 4104)])
+def test_unaligned_weights(M, N, K):
+    """W at an 8-byte address: 64 rows a launch, one of them short, with and without K splits."""
+    import torch
+
+    pool = (torch.randn(N * K + 4, device="cuda") * 0.02).bfloat16()
+    w = pool[4:].view(N, K)
+    assert w.data_ptr() % 16 == 8
+    x, b = torch.randn(M, K, device="cuda"), torch.randn(N, device="cuda").bfloat16()
+    y = torch.full((M + 1, N), 7.0, device="cuda")
+    R.linear(w.data_ptr(), x.data_ptr(), y.data_ptr(), M, N, K, b.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    ref = x.double() @ w.double().t() + b.double()
+    size = x.double().abs() @ w.double().abs().t() + b.double().abs()
+    assert float(((y[:M].double() - ref).abs() / size).max()) <= 2.0**-16 + K * 2.0**-24
+    assert bool((y[M] == 7).all())
+
+
 def linear_call(w, x, y, stream):
     R.linear(w.data_ptr(), x.data_ptr(), y.data_ptr(), x.shape[0], w.shape[0], w.shape[1], None, stream.cuda_stream)
 

@@ -71,3 +71,12 @@ def test_without_memory_for_partial_sums():
                 assert l.scratch_bytes == 0
             if kernel(e) == kernel(l):
                 assert l.scratch_bytes <= e.scratch_bytes
+
+
+def test_unaligned_weights_stay_off_the_copies():
+    """No kernel that copies W into LDS in 16-byte units gets a W at another address."""
+    for M in ROWS:
+        for N, K in SIZES:
+            r = R.linear_route(M, N, K, unaligned=True)
+            assert kernel(r) in ("gemv", "skinny"), (M, N, K)
+            assert r.scratch_bytes <= 64 * 1024 + 8 * 64 * N * 4

@@ -418,13 +418,15 @@ struct LinearPlan {
 
 size_t linear_plane_bytes(uint32_t M, uint32_t K) { return gemm_split_elems(M, K) * sizeof(uint16_t); }
 
-// aligned: W and X are at 16-byte addresses. lean: without partial sums, as a
-// call that cannot have more scratch runs.
-LinearPlan linear_plan(uint32_t M, uint32_t N, uint32_t K, bool aligned, bool lean, uint32_t cus) {
+// w_aligned, x_aligned: at 16-byte addresses, as the copies into LDS take them
+// (all of W, and the few-row GEMM's of X); the skinny kernel's loads do not ask
+// for it. lean: without partial sums, as a call that cannot have more scratch
+// runs.
+LinearPlan linear_plan(uint32_t M, uint32_t N, uint32_t K, bool w_aligned, bool x_aligned, bool lean, uint32_t cus) {
     LinearPlan p;
     if (linear_uses_gemv(M, N, K)) return p;
     const size_t sums = (size_t)M * N * sizeof(float);
-    if (M <= kSlabMaxRows && aligned && !lean) {
+    if (M <= kSlabMaxRows && w_aligned && x_aligned && !lean) {
         const PlainGemmPlan g = gemm_plain_plan(M, N, K, cus);
         if (g.few_rows && (M > kSkinnyMaxRows || slab_beats_skinny(M, N, K, g.splits, cus))) {
             p.kernel = LinearKernel::FewRows, p.splits = g.splits;
@@ -432,9 +434,9 @@ LinearPlan linear_plan(uint32_t M, uint32_t N, uint32_t K, bool aligned, bool le
             return p;
         }
     }
-    if (M <= kSkinnyMaxRows) {
+    if (M <= kSkinnyMaxRows || !w_aligned) {  // (more rows: a launch for every 64)
         p.kernel = LinearKernel::Skinny, p.splits = skinny_splits(N, K);
-        p.payload = p.splits > 1 ? p.splits * sums : 0;
+        p.payload = p.splits > 1 ? (size_t)p.splits * std::min(M, kSkinnyMaxRows) * N * sizeof(float) : 0;
         return p;
     }
     p.kernel = LinearKernel::Tiles, p.payload = linear_plane_bytes(M, K);
@@ -446,8 +448,8 @@ LinearPlan linear_plan(uint32_t M, uint32_t N, uint32_t K, bool aligned, bool le
 }
 
 LinearPlan linear_plan(const uint16_t* dW, const float* dX, uint32_t M, uint32_t N, uint32_t K, bool lean = false) {
-    const bool aligned = (reinterpret_cast<uintptr_t>(dW) | reinterpret_cast<uintptr_t>(dX)) % 16 == 0;
-    return linear_plan(M, N, K, aligned, lean, gemm_cus());
+    return linear_plan(M, N, K, reinterpret_cast<uintptr_t>(dW) % 16 == 0, reinterpret_cast<uintptr_t>(dX) % 16 == 0, lean,
+                       gemm_cus());
 }
 
 // Under capture a call that can do without scratch does, so that its graph
@@ -461,7 +463,9 @@ int linear_enqueue(const LinearPlan& p, const uint16_t* dW, const float* dX, con
     if (p.kernel == LinearKernel::Skinny) {
         float* ws = scratch_mem ? reinterpret_cast<float*>(scratch_mem + kCounterBytes) : nullptr;
         uint32_t* cnt = reinterpret_cast<uint32_t*>(scratch_mem);
-        HIP_TRY(launch_skinny(dW, dX, dBias, dY, M, N, K, ws, cnt, s));
+        for (uint32_t m = 0; m < M; m += kSkinnyMaxRows)
+            HIP_TRY(launch_skinny(dW, dX + static_cast<size_t>(m) * K, dBias, dY + static_cast<size_t>(m) * N,
+                                  std::min(M - m, kSkinnyMaxRows), N, K, ws, cnt, s));
         return VVLI_OK;
     }
     if (p.kernel == LinearKernel::FewRows || p.kernel == LinearKernel::Tiles) {
@@ -615,9 +619,10 @@ int vvli_gpu_linear_noalloc(const uint16_t* dW, const float* dX, const uint16_t*
                             uint32_t N, uint32_t K, void* stream) {
     int rc = check_linear_args(dW, dX, dY, M, N, K, "vvli_gpu_linear_noalloc");
     if (rc) return rc;
-    // (The bound that callers know is that of the lean plan: M > 64 its planes.)
+    // (The bound that callers know is that of aligned calls without partial
+    // sums: M > 64 their planes.)
     LinearPlan p = linear_plan(dW, dX, M, N, K);
-    const LinearPlan lean = linear_plan(dW, dX, M, N, K, true);
+    const LinearPlan lean = linear_plan(M, N, K, true, true, true, gemm_cus());
     const size_t bound = std::max(p.payload, lean.payload);
     if (bound > kNoAllocScratchBytes)
         return set_error(VVLI_INVALID_CONFIG,
@@ -632,10 +637,11 @@ int vvli_gpu_linear_noalloc(const uint16_t* dW, const float* dX, const uint16_t*
 int vvli_gpu_test_linear_route(uint32_t M, uint32_t N, uint32_t K, uint32_t cus, uint32_t flags,
                                vvli_gpu_linear_route* out) {
     if (!out) return set_error(VVLI_NULL_ARG, "NULL argument to vvli_gpu_test_linear_route");
-    if (M == 0 || N == 0 || K == 0 || K % 8 != 0 || cus == 0 || flags > (VVLI_ROUTE_CAPTURED | VVLI_ROUTE_LEAN))
+    if (M == 0 || N == 0 || K == 0 || K % 8 != 0 || cus == 0 || flags > (VVLI_ROUTE_CAPTURED | VVLI_ROUTE_LEAN | VVLI_ROUTE_UNALIGNED))
         return set_error(VVLI_INVALID_CONFIG, "bad linear route M=%u N=%u K=%u cus=%u", M, N, K, cus);
-    LinearPlan p = linear_plan(M, N, K, true, (flags & VVLI_ROUTE_LEAN) != 0, cus);
-    if (flags & VVLI_ROUTE_CAPTURED) p = captured_plan(p, linear_plan(M, N, K, true, true, cus));
+    const bool aligned = !(flags & VVLI_ROUTE_UNALIGNED);
+    LinearPlan p = linear_plan(M, N, K, aligned, true, (flags & VVLI_ROUTE_LEAN) != 0, cus);
+    if (flags & VVLI_ROUTE_CAPTURED) p = captured_plan(p, linear_plan(M, N, K, aligned, true, true, cus));
     out->kernel = static_cast<uint32_t>(p.kernel);
     out->splits = p.splits;
     out->gemm_few_rows = gemm_plain_plan(M, N, K, cus).few_rows;

@@ -414,10 +414,11 @@ def linear(dW: int, dX: int, dY: int, M: int, N: int, K: int, dBias: int | None 
 LINEAR_KERNELS = ("gemv", "skinny", "few_rows", "tiles")
 
 
-def linear_route(M: int, N: int, K: int, cus: int = 256, captured: bool = False, lean: bool = False) -> _lib.CLinearRoute:
+def linear_route(M: int, N: int, K: int, cus: int = 256, captured: bool = False, lean: bool = False,
+                 unaligned: bool = False) -> _lib.CLinearRoute:
     """vvli_gpu_test_linear_route: what ``linear`` runs on a device of ``cus`` compute units (no GPU needed)."""
     out = _lib.CLinearRoute()
-    _lib.check(_lib.lib().vvli_gpu_test_linear_route(M, N, K, cus, captured + 2 * lean, byref(out)))
+    _lib.check(_lib.lib().vvli_gpu_test_linear_route(M, N, K, cus, captured + 2 * lean + 4 * unaligned, byref(out)))
     return out
 
 
