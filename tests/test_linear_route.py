@@ -80,3 +80,23 @@ def test_unaligned_weights_stay_off_the_copies():
             r = R.linear_route(M, N, K, unaligned=True)
             assert kernel(r) in ("gemv", "skinny"), (M, N, K)
             assert r.scratch_bytes <= 64 * 1024 + 8 * 64 * N * 4
+
+
+# Timed on both sides (us: skinny or tiles / few-row GEMM): well away from the
+# lines between the kernels.
+@pytest.mark.parametrize("M,N,K,want", [
+    (64, 5000, 520, "skinny"),     # 8.6 / 11.6: short rows of X that don't start on cache lines
+    (64, 1927, 1136, "skinny"),    # 9.0 / 10.8
+    (5, 2048, 2048, "skinny"),     # 6.0 / 8.2
+    (16, 2048, 8192, "few_rows"),  # 22.9 / 11.6
+    (16, 9000, 3000, "few_rows"),  # 31.8 / 19.6
+    (5, 50304, 2048, "few_rows"),  # 57.6 / 40.4
+    (64, 512, 2048, "few_rows"),   # 18.4 / 9.2
+    (65, 3584, 18944, "tiles"),    # 54.4 / 68.1: 74 K chunks a block
+    (100, 11008, 4096, "tiles"),   # 43.4 / 58.7
+    (128, 18944, 3584, "tiles"),   # 61.2 / 101.8: two rounds
+    (65, 2048, 16384, "few_rows"), # 39.4 / 35.0: 32 chunks
+    (128, 8192, 2048, "few_rows"), # 29.2 / 25.3
+])
+def test_the_faster_kernel(M, N, K, want):
+    assert kernel(R.linear_route(M, N, K)) == want

@@ -8,6 +8,7 @@
 // its own for calls under capture), vvli_gpu_linear_noalloc uses a static
 // device array and allocates nothing.
 #include <algorithm>
+#include <cmath>
 #include <mutex>
 #include <utility>
 #include <vector>
@@ -386,22 +387,31 @@ bool linear_uses_gemv(uint32_t M, uint32_t N, uint32_t K) {
 // of gemm_slab.hpp stages X in LDS once per 64 rows of W where the skinny
 // kernel fetches it from L2 for every 16 to 64, but splits K across blocks with
 // a second launch that adds the splits; its copies need 16-byte aligned
-// pointers. Up to 64 rows the cheaper of the two by these estimates (us, fitted
-// to both kernels over ten shapes and M = 5 .. 64, within 20 %): a block of the
-// skinny kernel moves about 40 KB per us; a chunk of the few-row GEMM takes
-// kChunkUs. Measured, skinny / few-row: 2048 x 8192 M = 16 22.2 / 11.4, M = 64
-// 44.7 / 16.0; 128256 x 2048 M = 16 132.7 / 96; 2048 x 2048 M = 8 6.4 / 7.7,
-// M = 33 12.8 / 9.5; 1152 x 896 M = 33 7.0 / 8.0. From 65 to 128 rows what
-// gemm_plain_plan takes, against the split pass and the tiles: 2048 x 2048 M =
-// 96 21.8 / 13.7; 8192 x 2048 M = 128 34.7 / 25.5.
+// pointers. Up to 64 rows the cheaper of the two by these estimates (us; both
+// kernels timed at 73 shapes and 13 or 14 row counts from 4 to 64, skinny
+// within 12 % of its estimate, few-row within 8 %; the rule's choice is on
+// average 0.8 % slower than the faster kernel, 2.3 % with one rate for all
+// shapes, which took the few-row GEMM for 64 x 5000 x 520 at 11.6 us against
+// 8.6):
+//   skinny: its blocks move X and W at a rate (KB per us) that falls with the
+//   rows of W a block has (16, 32, 64) and is higher where X's rows don't start
+//   on cache lines (K % 32) and are short: those spread over the L2 channels.
+//   Blocks share CUs unevenly except in that case.
+//   few-row: kChunkUs per K chunk of a block, and its split sums.
+// Measured, skinny / few-row: 2048 x 8192 M = 16 22.9 / 11.6, M = 64 45.3 /
+// 16.0; 128256 x 2048 M = 16 132.7 / 89.5; 2048 x 2048 M = 5 6.0 / 8.2, M = 32
+// 11.6 / 9.2; 1152 x 896 M = 32 6.4 / 7.9; 1927 x 1136 M = 48 7.6 / 10.3. From
+// 65 to 128 rows what gemm_plain_plan takes.
 bool slab_beats_skinny(uint32_t M, uint32_t N, uint32_t K, uint32_t slab_splits, uint32_t cus) {
-    const float rows = static_cast<float>(M), k = static_cast<float>(K);
-    const uint32_t ks0 = skinny_splits(N, K), blocks = skinny_tiles(N) * ks0;
-    const float skinny = 2.8f + (ks0 > 1 ? 5.f : 0.f) +
-                         static_cast<float>((blocks + cus - 1) / cus) * (k / ks0) * (4.f * rows + 32.f * skinny_nt(N)) / 40e3f;
-    constexpr float kChunkUs[] = {0.5f, 0.65f, 0.95f, 0.95f};  // 16, 32, 64 rows
+    const uint32_t ks0 = skinny_splits(N, K), blocks = skinny_tiles(N) * ks0, nt = skinny_nt(N);
+    const float per_cu = static_cast<float>(blocks) / cus;
+    const bool spread = nt == 1 && K % 32 != 0 && K <= 2304 * ks0;
+    const float rate = spread ? (blocks <= cus ? 46e3f : 30e3f) : nt == 1 ? 36e3f : nt == 2 ? 32e3f : 26e3f;
+    const float rounds = spread ? std::max(1.f, per_cu) : std::ceil(per_cu);
+    const float skinny = 2.7f + (ks0 > 1 ? 7.f : 0.f) + rounds * (static_cast<float>(K) / ks0) * (4.f * M + 32.f * nt) / rate;
+    constexpr float kChunkUs[] = {0.53f, 0.66f, 1.f, 1.f};  // 16, 32, 64 rows
     const uint32_t ks = slab_splits, tiles = (N + 63) / 64, chunks = ((K + 127) / 128 + ks - 1) / ks;
-    const float slab = 4.4f + (ks > 1 ? 2.6f : 0.f) +
+    const float slab = 5.5f + (ks > 1 ? 1.3f + 0.7f * 4e-6f * ks * M * N : 0.f) +
                        static_cast<float>((tiles * ks + cus - 1) / cus * chunks) * kChunkUs[(M - 1) / 16];
     return slab < skinny;
 }

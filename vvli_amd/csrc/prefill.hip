@@ -1356,12 +1356,16 @@ static GemmPlan gemm_plan(int mode, const GemmArgs& g, uint32_t cus) {
     // Few rows: the slab kernel. Up to 64 rows always (one layer of the 1B
     // shape at 45 rows: gate/up 36 -> 20 us with its zeroing and SwiGLU passes,
     // o and down 17 -> 9.5, q|k|v 15 -> 9.5); from 65 to 128 while its items
-    // are one round (8192 x 2048 at 128 rows 25.5 us against 34.7 on the
-    // tiles, 18944 x 3584 102 against 61).
+    // are one round of at most 40 K chunks (linear at 65 / 128 rows, us, this
+    // and the tiles with their split pass: 8192 x 2048 23.7 / 25.3 and 25.8 /
+    // 29.2; 16384 x 2560, 40 chunks, 40.3 / 41.9 and 37.0 / 44.4; 4096 x 11008,
+    // 43 chunks, 44.1 / 45.8 and 38.5 / 44.9; 3584 x 18944, 74 chunks, 68.1 /
+    // 69.1 and 54.4 / 57.2; 18944 x 3584, two rounds, 101 / 102 and 54 / 61).
     if (g.M <= kSlabMaxRows && (mode != kGemmPlain || g.ldo == g.N || !g.part)) {
         const uint32_t tiles = (cols + kSlabN - 1) / kSlabN;
         const uint32_t splits = mode != kGemmGateUp && g.part ? slab_splits(tiles, g.K, g.M, cus) : 1u;
-        if (g.M <= 64 || tiles * splits <= cus) return {GemmKernel::Slab, splits};
+        const uint32_t chunks = ((g.K + 63) / 64 + splits - 1) / splits;
+        if (g.M <= 64 || (tiles * splits <= cus && chunks <= 40)) return {GemmKernel::Slab, splits};
     }
     const uint32_t gx = (cols + kBN - 1) / kBN, gy = (g.M + kBM - 1) / kBM;
     const uint32_t splits = gemm_k_splits(mode, g, gx * gy, cus);
