@@ -270,7 +270,8 @@ int vvli_gpu_profile_step(vvli_gpu_model* model, uint32_t token, uint32_t pos, f
  * checking both against the same reference. */
 int vvli_gpu_set_decode_path(vvli_gpu_model* model, uint32_t path);
 /* How vvli_gpu_prefill (and generate with VVLI_GEN_BATCHED_PREFILL) runs the
- * prompt: 0 = auto (batched where supported; f32 weights in f32 throughout),
+ * prompt: 0 = auto (batched where supported; f32 weights in f32 throughout,
+ * from two rows on unless they are few behind a long cache),
  * 1 = token loop, 2 = batched with bf16 weights (VVLI_INVALID_CONFIG if the
  * model does not support it). */
 int vvli_gpu_set_prefill_path(vvli_gpu_model* model, uint32_t path);
@@ -309,6 +310,10 @@ int vvli_gpu_test_inject_step_error(vvli_gpu_model* model, uint32_t n);
  * Form 2 needs heads / kv_heads <= 64 (else the prefill returns
  * VVLI_HIP_ERROR). Values outside -1..2 -> VVLI_INVALID_CONFIG. */
 int vvli_gpu_test_set_prefill_attention_form(int32_t form);
+/* Test hook of the batched prefill (needs no GPU): 1 if a prompt of n rows
+ * behind `start` cached ones takes it under vvli_gpu_set_prefill_path(0), 0 if
+ * it takes the token loop. */
+int vvli_gpu_test_prefill_batched(const vvli_gpu_config* cfg, uint32_t start, uint32_t n);
 /* Test hook of the whole-vocabulary sampler (no reference counterpart):
  * Sampler.next as vvli_gpu_sampler_next with no repeat history, restricted to
  * candidate lists over 1024 (temperature > 0, top_k 0 or > 1024; else

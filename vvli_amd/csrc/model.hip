@@ -760,13 +760,31 @@ bool prefill_f32_supported(const vvli_gpu_config& c) {
     return c.weight_kind == VVLI_WEIGHT_F32 && (hd == 32 || hd == 64 || hd == 128);
 }
 
+// Whether n f32 rows behind `start` cached ones go through it: each row past
+// the first saves a token step, while a short prompt's attention walks all keys
+// in a few blocks, where the token step splits them over the CUs. One row: the
+// token step. Measured, ms, token loop / batched: Qwen2.5-0.5B (60 MB a layer)
+// 2 rows 2.33 / 1.04, behind 4000 3.03 / 2.65, behind 6000 3.35 / 3.44, behind
+// 32000 6.3 / 14; 3 behind 9000 5.67 / 4.60, behind 12000 5.87 / 5.78; eight
+// layers of width 512 (16 MB) 2 rows 0.51 / 0.28, behind 4000 0.68 / 0.78, of
+// width 256 (2.4 MB) 2 behind 4000 0.56 / 0.76. One row 1.17 / 1.01 there, but
+// 0.36 / 0.38 through four Llama-3.2-1B layers, 0.44 / 0.51 through two of
+// Qwen2.5-7B, and behind 32000 0.54 / 2.32 (four of Qwen2.5-0.5B's).
+bool prefill_f32_batched(const vvli_gpu_config& c, uint32_t start, uint32_t n) {
+    const uint64_t kv = kv_dim(c), layer_mb = (4ull * c.hidden * (2ull * c.hidden + 2 * kv + 3ull * c.inter)) >> 20;
+    const uint64_t keys = std::min<uint64_t>(5000, 1500 + 60 * layer_mb);  // what a token step is worth
+    return n > 1 && start <= (n - 1) * keys;
+}
+
 int ensure_prefill_buffers(vvli_gpu_model* m);
 
-bool use_batched_prefill(vvli_gpu_model* m) {
+bool use_batched_prefill(vvli_gpu_model* m, uint32_t start, uint32_t n) {
     if (m->prefill_path == 1) return false;
     if (prefill_supported(m->cfg)) return true;
     // The token loop needs no chunk buffers: it serves where they do not fit.
-    if (!prefill_f32_supported(m->cfg) || hipSetDevice(m->device) != hipSuccess) return false;
+    if (!prefill_f32_supported(m->cfg) || !prefill_f32_batched(m->cfg, start, n) ||
+        hipSetDevice(m->device) != hipSuccess)
+        return false;
     if (ensure_prefill_buffers(m) == VVLI_OK) return true;
     (void)hipGetLastError();  // (else the loop's first launch would report it)
     return false;
@@ -1851,6 +1869,11 @@ int vvli_gpu_kv_read(vvli_gpu_model* m, uint32_t layer, uint32_t pos, float* k_o
     return VVLI_OK;
 }
 
+int vvli_gpu_test_prefill_batched(const vvli_gpu_config* cfg, uint32_t start, uint32_t n) {
+    if (!cfg) return 0;
+    return prefill_supported(*cfg) || (prefill_f32_supported(*cfg) && prefill_f32_batched(*cfg, start, n));
+}
+
 int vvli_gpu_prefill(vvli_gpu_model* m, const uint32_t* tokens, uint32_t n, uint32_t start_pos, float* last_logits,
                      uint32_t* argmax_out) {
     if (!m || !tokens) return set_error(VVLI_NULL_ARG, "NULL argument to vvli_gpu_prefill");
@@ -1863,7 +1886,7 @@ int vvli_gpu_prefill(vvli_gpu_model* m, const uint32_t* tokens, uint32_t n, uint
     RESIDENT_STOP(m);
     // Prompt tokens live at their absolute positions in `prompt`.
     HIP_TRY(hipMemcpyAsync(m->prompt + start_pos, tokens, n * sizeof(uint32_t), hipMemcpyHostToDevice, m->stream));
-    if (use_batched_prefill(m)) {
+    if (use_batched_prefill(m, start_pos, n)) {
         int rc = enqueue_prefill_batched(m, start_pos, n, tokens[n - 1], 0);
         if (rc) return rc;
         return read_outputs(m, last_logits, argmax_out);
@@ -1889,7 +1912,7 @@ int vvli_gpu_generate_greedy(vvli_gpu_model* m, const uint32_t* prompt, uint32_t
         if (prompt[i] >= m->cfg.vocab) return set_error(VVLI_INVALID_TOKEN, "prompt token %u >= vocab", prompt[i]);
     if (n_prompt > m->max_seq)
         return set_error(VVLI_CONTEXT_FULL, "prompt of %u tokens > max_seq_len %u", n_prompt, m->max_seq);
-    const bool batched = (flags & VVLI_GEN_BATCHED_PREFILL) && use_batched_prefill(m);
+    const bool batched = (flags & VVLI_GEN_BATCHED_PREFILL) && use_batched_prefill(m, 0, n_prompt);
     HIP_TRY(hipSetDevice(m->device));
     RESIDENT_STOP(m);
     if (use_persistent(m))
@@ -1962,7 +1985,7 @@ int vvli_gpu_generate(vvli_gpu_model* m, const uint32_t* prompt, uint32_t n_prom
         return set_error(VVLI_CONTEXT_FULL, "prompt of %u tokens > max_seq_len %u", n_prompt, m->max_seq);
     HIP_TRY(hipSetDevice(m->device));
     RESIDENT_STOP(m);
-    const bool batched = (flags & VVLI_GEN_BATCHED_PREFILL) && use_batched_prefill(m);
+    const bool batched = (flags & VVLI_GEN_BATCHED_PREFILL) && use_batched_prefill(m, 0, n_prompt);
     return generate_sampled(m, prompt, n_prompt, max_new, eos, batched, *opts, out_tokens, n_out, stats);
 }
 
