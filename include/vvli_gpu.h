@@ -314,6 +314,10 @@ int vvli_gpu_test_set_prefill_attention_form(int32_t form);
  * behind `start` cached ones takes it under vvli_gpu_set_prefill_path(0), 0 if
  * it takes the token loop. */
 int vvli_gpu_test_prefill_batched(const vvli_gpu_config* cfg, uint32_t start, uint32_t n);
+/* Test hook of the batched prefill: its chunk buffers (not yet allocated) may
+ * take at most `bytes` from now on, as if the device had no more. *tries_out
+ * (or NULL) = how often they were asked for so far. */
+int vvli_gpu_test_limit_prefill_memory(vvli_gpu_model* model, size_t bytes, uint32_t* tries_out);
 /* Test hook of the whole-vocabulary sampler (no reference counterpart):
  * Sampler.next as vvli_gpu_sampler_next with no repeat history, restricted to
  * candidate lists over 1024 (temperature > 0, top_k 0 or > 1024; else

@@ -88,3 +88,32 @@ def test_f32_generation_and_paths(oracle_mod):
         a, _ = gpu.generate_greedy_measured(prompt, 12, batched_prefill=True)
         b, _ = gpu.generate_greedy_measured(prompt, 12, batched_prefill=False)
         assert a.tolist() == b.tolist()
+
+
+def test_f32_prefill_without_room_for_its_buffers():
+    """Prompts whose chunk buffers do not fit run the token loop, report no
+    error, ask for the memory once, and take the batched prefill when there is
+    room again."""
+    from ctypes import byref, c_uint32
+
+    from vvli_amd import _lib
+
+    c = cfg()
+    blob = R.synthetic_blob(c, C.WEIGHT_F32, seed=2, stddev=0.05)
+    prompt = np.arange(5, 45, dtype=np.uint32)
+    tries = c_uint32()
+
+    def limit(gpu, n) -> int:
+        _lib.check(_lib.lib().vvli_gpu_test_limit_prefill_memory(gpu._h, n, byref(tries)))
+        return tries.value
+
+    with R.Runner(c, blob, 64) as gpu, R.Runner(c, blob, 64) as loop:
+        loop.set_prefill_path("loop")
+        want = loop.prefill(prompt)[0].copy()
+        limit(gpu, 1000)
+        for _ in range(3):
+            assert np.array_equal(gpu.prefill(prompt)[0], want)  # the same token loop
+        assert limit(gpu, 2**63) == 1
+        assert rel_err(gpu.prefill(prompt)[0], want) <= TOL
+        gpu.prefill(prompt)
+        assert limit(gpu, 2**63) == 2

@@ -101,6 +101,9 @@ struct vvli_gpu_model {
     bool pf_ok = false;
     uint32_t prefill_path = 0;  // 0 auto, 1 token loop, 2 batched
     uint32_t pf_rows = 0;       // rows per chunk the buffers hold
+    size_t pf_wanted = 0;       // bytes of the chunk buffers when they last did not fit
+    size_t pf_limit = SIZE_MAX; // (test hook: bytes they may take)
+    uint32_t pf_tries = 0;      // (test hook: times they were asked for)
     float* pf_x = nullptr;      // [rows][H] residual stream
     float* pf_qkv = nullptr;    // [rows][H + 2 kv]
     float* pf_attn = nullptr;   // [rows][H]
@@ -785,6 +788,13 @@ bool use_batched_prefill(vvli_gpu_model* m, uint32_t start, uint32_t n) {
     if (!prefill_f32_supported(m->cfg) || !prefill_f32_batched(m->cfg, start, n) ||
         hipSetDevice(m->device) != hipSuccess)
         return false;
+    if (m->pf_wanted) {  // not asked for again before there is room
+        size_t free_bytes = 0, total = 0;
+        if (hipMemGetInfo(&free_bytes, &total) != hipSuccess || std::min(free_bytes, m->pf_limit) < m->pf_wanted) {
+            (void)hipGetLastError();
+            return false;
+        }
+    }
     if (ensure_prefill_buffers(m) == VVLI_OK) return true;
     (void)hipGetLastError();  // (else the loop's first launch would report it)
     return false;
@@ -798,8 +808,14 @@ int ensure_prefill_buffers(vvli_gpu_model* m) {
     float** bufs[] = {&m->pf_x, &m->pf_qkv, &m->pf_attn, &m->pf_scale, &m->pf_ahl, &m->pf_ahl2};
     const size_t split = (gemm_split_elems(static_cast<uint32_t>(rows), static_cast<uint32_t>(std::max(H, I))) + 1) / 2;
     const size_t sizes[] = {rows * H, rows * (H + 2 * kv), rows * H, rows, split, split};
+    const bool f32 = c.weight_kind == VVLI_WEIGHT_F32;  // (its attention reads the cache rows themselves)
+    const size_t kvp = f32 ? 0 : prefill_kv_pack_bytes(static_cast<uint32_t>(m->max_seq), c.kv_heads, head_dim(c));
+    m->pf_wanted = kvp;
+    for (size_t n : sizes) m->pf_wanted += n * sizeof(float);
+    ++m->pf_tries;
     for (int i = 0; i < 6; ++i) {
-        hipError_t e = hipMalloc(reinterpret_cast<void**>(bufs[i]), sizes[i] * sizeof(float));
+        hipError_t e = m->pf_wanted > m->pf_limit ? hipErrorOutOfMemory
+                                                  : hipMalloc(reinterpret_cast<void**>(bufs[i]), sizes[i] * sizeof(float));
         if (e != hipSuccess) {
             for (float** b : bufs) {
                 if (*b) (void)hipFree(*b);
@@ -809,8 +825,6 @@ int ensure_prefill_buffers(vvli_gpu_model* m) {
                              "prefill buffers (%zu rows): %s", rows, hipGetErrorString(e));
         }
     }
-    const bool f32 = c.weight_kind == VVLI_WEIGHT_F32;  // (its attention reads the cache rows themselves)
-    const size_t kvp = f32 ? 0 : prefill_kv_pack_bytes(static_cast<uint32_t>(m->max_seq), c.kv_heads, head_dim(c));
     hipError_t e = f32 ? hipSuccess : hipMalloc(&m->pf_kvp, kvp);
     if (e != hipSuccess) {
         for (float** b : bufs) {
@@ -821,6 +835,7 @@ int ensure_prefill_buffers(vvli_gpu_model* m) {
         return set_error(e == hipErrorOutOfMemory ? VVLI_OUT_OF_MEMORY : VVLI_HIP_ERROR,
                          "prefill K/V tiles (%zu bytes): %s", kvp, hipGetErrorString(e));
     }
+    m->pf_wanted = 0;
     m->pf_kvp_bytes = kvp;
     m->pf_rows = static_cast<uint32_t>(rows);
     e = hipMalloc(reinterpret_cast<void**>(&m->pf_part), gemm_part_elems() * sizeof(float));
@@ -1866,6 +1881,13 @@ int vvli_gpu_kv_read(vvli_gpu_model* m, uint32_t layer, uint32_t pos, float* k_o
     if (v_out)
         HIP_TRY(hipMemcpyAsync(v_out, m->vcache + off, kv * sizeof(float), hipMemcpyDeviceToHost, m->stream));
     HIP_TRY(hipStreamSynchronize(m->stream));
+    return VVLI_OK;
+}
+
+int vvli_gpu_test_limit_prefill_memory(vvli_gpu_model* m, size_t bytes, uint32_t* tries_out) {
+    if (!m) return set_error(VVLI_NULL_ARG, "NULL argument to vvli_gpu_test_limit_prefill_memory");
+    m->pf_limit = bytes;
+    if (tries_out) *tries_out = m->pf_tries;
     return VVLI_OK;
 }
 
