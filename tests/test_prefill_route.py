@@ -23,8 +23,10 @@ def batched(cfg, start, n, kind=C.WEIGHT_F32) -> bool:
     (C.NAMED["qwen2.5-0.5b"](), 0, 2, True),        # 2.33 / 1.04
     (C.NAMED["qwen2.5-0.5b"](), 4000, 2, True),     # 3.03 / 2.65
     (C.NAMED["qwen2.5-0.5b"](), 16000, 2, False),   # 0.77 / 1.27 (four layers)
+    (C.NAMED["qwen2.5-0.5b"](), 16000, 4, True),    # 1.51 / 1.22 (four layers)
     (C.NAMED["qwen2.5-0.5b"](), 32000, 4, False),   # 2.08 / 2.31 (four layers)
-    (C.NAMED["qwen2.5-0.5b"](), 32000, 8, True),    # 4.13 / 2.30 (four layers)
+    (C.NAMED["qwen2.5-0.5b"](), 32000, 6, True),    # 3.11 / 2.30 (four layers)
+    (C.NAMED["qwen2.5-0.5b"](), 32000, 2**31, True),
     (C.NAMED["llama-3.2-1b"](), 0, 1, False),       # 0.36 / 0.38 (four layers)
     (C.NAMED["llama-3.2-1b"](), 2000, 1, False),    # 0.39 / 0.51 (four layers)
     (C.NAMED["llama-3.2-1b"](), 2000, 2, True),     # 0.74 / 0.51 (four layers)
@@ -33,6 +35,7 @@ def batched(cfg, start, n, kind=C.WEIGHT_F32) -> bool:
     (NARROW, 0, 2, True),                           # 0.42 / 0.26 (eight layers)
     (NARROW, 4000, 2, False),                       # 0.56 / 0.76 (eight layers)
     (NARROW, 14000, 4, False),                      # 1.47 / 2.00 (eight layers)
+    (NARROW, 24000, 6, False),                      # 2.62 / 3.25 (eight layers)
     (NARROW, 100, 33, True),
 ])
 def test_f32_prompts(cfg, start, n, want):

@@ -765,18 +765,20 @@ bool prefill_f32_supported(const vvli_gpu_config& c) {
 
 // Whether n f32 rows behind `start` cached ones go through it: each row past
 // the first saves a token step, while a short prompt's attention walks all keys
-// in a few blocks, where the token step splits them over the CUs. One row: the
-// token step. Measured, ms, token loop / batched: Qwen2.5-0.5B (60 MB a layer)
-// 2 rows 2.33 / 1.04, behind 4000 3.03 / 2.65, behind 6000 3.35 / 3.44, behind
-// 32000 6.3 / 14; 3 behind 9000 5.67 / 4.60, behind 12000 5.87 / 5.78; eight
+// in a few blocks, where the token step splits them over the CUs (but walks
+// them again for every row). One row: the token step. Measured, ms, token loop
+// / batched: Qwen2.5-0.5B (60 MB a layer) 2 rows 2.33 / 1.04, behind 4000 3.03
+// / 2.65, behind 6000 3.35 / 3.44, behind 32000 6.3 / 14; 3 behind 9000 5.67 /
+// 4.60, behind 12000 5.87 / 5.78; 4 behind 18000 9.68 / 8.15; eight
 // layers of width 512 (16 MB) 2 rows 0.51 / 0.28, behind 4000 0.68 / 0.78, of
 // width 256 (2.4 MB) 2 behind 4000 0.56 / 0.76. One row 1.17 / 1.01 there, but
 // 0.36 / 0.38 through four Llama-3.2-1B layers, 0.44 / 0.51 through two of
 // Qwen2.5-7B, and behind 32000 0.54 / 2.32 (four of Qwen2.5-0.5B's).
 bool prefill_f32_batched(const vvli_gpu_config& c, uint32_t start, uint32_t n) {
     const uint64_t kv = kv_dim(c), layer_mb = (4ull * c.hidden * (2ull * c.hidden + 2 * kv + 3ull * c.inter)) >> 20;
-    const uint64_t keys = std::min<uint64_t>(5000, 1500 + 60 * layer_mb);  // what a token step is worth
-    return n > 1 && start <= (n - 1) * keys;
+    const uint64_t keys = std::min<uint64_t>(5000, 1300 + 64 * layer_mb);  // even at two rows
+    const uint64_t r = std::min(n, 64u);
+    return r > 1 && start <= keys * (r - 1) * (r + 3) / 5;
 }
 
 int ensure_prefill_buffers(vvli_gpu_model* m);
