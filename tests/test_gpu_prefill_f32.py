@@ -117,3 +117,27 @@ def test_f32_prefill_without_room_for_its_buffers():
         assert rel_err(gpu.prefill(prompt)[0], want) <= TOL
         gpu.prefill(prompt)
         assert limit(gpu, 2**63) == 2
+
+
+@pytest.mark.parametrize("hd,heads,kv", [(64, 4, 2), (32, 7, 1), (128, 2, 2)])
+def test_f32_prefill_rows_before_a_nan_row(hd, heads, kv):
+    """A row that is NaN (its embedding is) leaves the rows before it as the
+    token loop does: hidden keys have no weight, whatever their values."""
+    c = cfg(hidden_size=hd * heads, num_attention_heads=heads, num_key_value_heads=kv)
+    blob = R.synthetic_blob(c, C.WEIGHT_F32, seed=4, stddev=0.05)
+    bad, at, n = 77, 25, 37  # (not the first row of a block of 16 query vectors)
+    blob[bad * c.hidden_size] = np.nan  # (the embedding comes first)
+    toks = np.arange(100, 100 + n, dtype=np.uint32)
+    toks[at] = bad
+    with R.Runner(c, blob, 64) as gpu, R.Runner(c, blob, 64) as loop:
+        loop.set_prefill_path("loop")
+        for r in (gpu, loop):
+            r.prefill(toks[:5], 0)
+            r.prefill(toks[5:], 5)
+        for layer in range(c.num_hidden_layers):
+            for pos in range(n):
+                for g, r in zip(gpu.kv_read(layer, pos), loop.kv_read(layer, pos)):
+                    assert np.array_equal(np.isnan(g), np.isnan(r)), f"layer {layer} pos {pos}"
+                    assert bool(np.isnan(r).all()) == (pos == at or (pos > at and layer > 0))
+                    if pos < at:
+                        assert rel_err(g, r) <= TOL

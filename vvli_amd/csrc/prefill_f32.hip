@@ -10,6 +10,7 @@
 // o_proj and down 9 on average, q|k|v 7; gate/up's bytes and products take 6
 // each), with two of a block's load groups in flight.
 #include <algorithm>
+#include <type_traits>
 
 #include "device_common.hpp"
 #include "kernels.hpp"
@@ -245,7 +246,11 @@ __global__ __launch_bounds__(256) void embed_rows_f32_kernel(const float* __rest
 // wave order. Products transposed, as in prefill.hip: S^T = K . Q^T gives lane
 // l the scores of keys 4 (l / 16) + j of vector l % 16, which are its operand
 // of O^T += V^T . P^T. K and V come from the caches; the next chunk's are
-// loaded while this one is multiplied.
+// loaded while this one is multiplied. A hidden key has weight 0, which its V
+// must not turn into NaN (a later row's V may be anything): the chunks with
+// hidden keys, which come last, take V's values that are not finite out of the
+// products and add them for the vectors that see them. (In a loop of their own:
+// the check in the loop over all chunks cost 5 % behind 16000 rows.)
 // ---------------------------------------------------------------------------
 template <int HD>
 __global__ __launch_bounds__(kF32Threads) void attn_f32_kernel(PrefillAttnArgs a) {
@@ -262,6 +267,7 @@ __global__ __launch_bounds__(kF32Threads) void attn_f32_kernel(PrefillAttnArgs a
     const uint32_t row = vec / G, head = kvh * G + vec % G, pos = a.start + row;
     const uint32_t keys = a.start + min(v0 + 15, nvec - 1) / G + 1;  // keys of the block's last vector
     const uint32_t chunks = (keys + 15) / 16;
+    const uint32_t first_pos = a.start + v0 / G;  // position of the block's first vector
 
     f32x4 q[DT], o[DT];
 #pragma unroll
@@ -288,8 +294,8 @@ __global__ __launch_bounds__(kF32Threads) void attn_f32_kernel(PrefillAttnArgs a
             for (int d = 0; d < DT; ++d) v[j][d] = *as_global(p + d * 16);
         }
     };
-    if (static_cast<uint32_t>(wave) < chunks) load_k(wave);
-    for (uint32_t c = wave; c < chunks; c += kF32Waves) {
+    auto chunk = [&](uint32_t c, auto hidden) {  // hidden: keys that some vector must not see
+        constexpr bool Hidden = decltype(hidden)::value;
         load_v(c);
         f32x4 s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -303,7 +309,7 @@ __global__ __launch_bounds__(kF32Threads) void attn_f32_kernel(PrefillAttnArgs a
         float mx = -INFINITY;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            s[j] = c * 16 + fq * 4 + j <= pos ? __fmul_rn(s[j], a.scale) : -INFINITY;
+            s[j] = !Hidden || c * 16 + fq * 4 + j <= pos ? __fmul_rn(s[j], a.scale) : -INFINITY;
             mx = fmaxf(mx, s[j]);
         }
         mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
@@ -317,15 +323,50 @@ __global__ __launch_bounds__(kF32Threads) void attn_f32_kernel(PrefillAttnArgs a
         for (int j = 0; j < 4; ++j) p[j] = expf(s[j] - ms), add += p[j];
         l = l * corr + add;
         m = mn;
+        bool strange = false;
+        if (Hidden) {
+            float t = 0.f;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int d = 0; d < DT; ++d) t = fmaf(v[j][d], 0.f, t);  // NaN if one is not finite
+            strange = __any(t != 0.f);
+            if (strange)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int d = 0; d < DT; ++d) v[j][d] = fabsf(v[j][d]) < INFINITY ? v[j][d] : 0.f;
+        }
         f32x4 add_o[DT];
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
             for (int d = 0; d < DT; ++d)
                 add_o[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[j][d], p[j], j ? add_o[d] : f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        if (strange) {  // p[i % 4] of key i sits in the lanes of group i / 4
+#pragma unroll 1
+            for (uint32_t i = 0; i < 16; ++i) {
+                const float pi = i & 2 ? (i & 1 ? p[3] : p[2]) : (i & 1 ? p[1] : p[0]);
+                const float pk = __shfl(pi, (i / 4) * 16 + fr, 64);
+                const uint32_t key = c * 16 + i;
+                const float* vp = a.vcache + static_cast<size_t>(min(key, keys - 1)) * a.kvdim + kvh * HD + fq * 4;
+#pragma unroll
+                for (int d = 0; d < DT; ++d) {
+                    const f32x4 x = *as_global(reinterpret_cast<const f32x4*>(vp + d * 16));
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (key <= pos && !(fabsf(x[e]) < INFINITY)) add_o[d][e] = fmaf(pk, x[e], add_o[d][e]);
+                    __builtin_amdgcn_sched_barrier(0);  // (few registers for a rare path)
+                }
+            }
+        }
 #pragma unroll
         for (int d = 0; d < DT; ++d) o[d] = o[d] * corr + add_o[d];
-    }
+    };
+    uint32_t c = wave;
+    if (c < chunks) load_k(c);
+    for (; c < chunks && c * 16 + 15 <= first_pos; c += kF32Waves) chunk(c, std::false_type{});
+    for (; c < chunks; c += kF32Waves) chunk(c, std::true_type{});
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
     if (fq == 0) sm[wave][fr] = m, sl[wave][fr] = l;
