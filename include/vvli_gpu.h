@@ -381,13 +381,13 @@ int vvli_gpu_linear_noalloc(const uint16_t* dW, const float* dX, const uint16_t*
 /* Test hook of vvli_gpu_linear (no reference counterpart; needs no GPU): what
  * a call runs on a device of `cus` compute units (flags: captured; lean, when
  * there is no memory for partial sums; dW not 16-byte aligned). kernel: 0 GEMV, 1 skinny, 2 few-row GEMM, 3 tiles; splits: of K;
- * gemm_few_rows: whether the prefill GEMM, given these sizes, would run its
- * few-row kernel; scratch_bytes: scratch of the call (0: none). */
+ * gemm_kernel: what the prefill GEMM runs at these sizes, 0 the 128 x 256 tile,
+ * 1 256 x 256, 2 its few-row kernel, 3 128 x 128; scratch_bytes: scratch of the call (0: none). */
 #define VVLI_ROUTE_CAPTURED 1u
 #define VVLI_ROUTE_LEAN 2u
 #define VVLI_ROUTE_UNALIGNED 4u
 typedef struct vvli_gpu_linear_route {
-    uint32_t kernel, splits, gemm_few_rows, reserved;
+    uint32_t kernel, splits, gemm_kernel, reserved;
     uint64_t scratch_bytes;
 } vvli_gpu_linear_route;
 int vvli_gpu_test_linear_route(uint32_t M, uint32_t N, uint32_t K, uint32_t cus, uint32_t flags,

@@ -16,9 +16,12 @@ from vvli_amd import runtime as R
 pytestmark = pytest.mark.gpu
 
 
-def check_linear(M, N, K, bias):
+def check_linear(M, N, K, bias, gemm_kernel):
     import torch
 
+    route = R.linear_route(M, N, K)
+    assert R.GEMM_KERNELS[route.gemm_kernel] == gemm_kernel  # the sizes still reach what they are here for
+    assert R.LINEAR_KERNELS[route.kernel] == ("few_rows" if gemm_kernel == "few_rows" else "tiles")
     g = torch.Generator(device="cuda").manual_seed(M * 31 + N * 7 + K)
     w = (torch.randn(N, K, device="cuda", generator=g) * 0.02).bfloat16()
     x = torch.randn(M, K, device="cuda", generator=g)
@@ -42,7 +45,14 @@ def check_linear(M, N, K, bias):
 @pytest.mark.parametrize("M,N,K,bias", [(512, 32768, 8, False), (511, 32741, 40, True), (385, 32760, 96, False),
                                         (500, 32513, 136, True), (2048, 8192, 256, False)])
 def test_wide_tile(M, N, K, bias):
-    check_linear(M, N, K, bias)
+    check_linear(M, N, K, bias, "256x256")
+
+
+# The 128 x 256 tile: unsplit, K split three ways (summed by a pass of their
+# own) and 32 ways (added atomically), ragged rows and columns.
+@pytest.mark.parametrize("M,N,K,bias", [(129, 18900, 64, True), (129, 9000, 2048, False), (130, 100, 8192, True)])
+def test_tile(M, N, K, bias):
+    check_linear(M, N, K, bias, "128x256")
 
 
 # The few-row GEMM: each row tile (16, 32, 64, 128 rows) with ragged rows and
@@ -53,7 +63,7 @@ def test_wide_tile(M, N, K, bias):
                                         (65, 200, 40, False), (100, 8200, 520, True), (128, 130, 72, True),
                                         (128, 2048, 8, False)])
 def test_few_rows(M, N, K, bias):
-    check_linear(M, N, K, bias)
+    check_linear(M, N, K, bias, "few_rows")
 
 
 def test_few_rows_unaligned_and_repeated():
@@ -252,7 +262,7 @@ def test_few_row_prefill():
                                         (512, 8192, 136, False), (512, 8190, 504, True), (300, 1000, 2056, True),
                                         (131, 1001, 4024, False), (700, 513, 8192, True)])
 def test_square_tile(M, N, K, bias):
-    check_linear(M, N, K, bias)
+    check_linear(M, N, K, bias, "128x128")
 
 
 def test_square_tile_prefill():

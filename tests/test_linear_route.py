@@ -23,10 +23,10 @@ def test_few_rows_only_where_the_gemm_takes_it(cus):
         for N, K in SIZES:
             r = R.linear_route(M, N, K, cus)
             if kernel(r) == "few_rows":
-                assert r.gemm_few_rows and M <= 128, (M, N, K, cus)
+                assert R.GEMM_KERNELS[r.gemm_kernel] == "few_rows" and M <= 128, (M, N, K, cus)
             elif M > 64:
                 assert kernel(r) == "tiles" and r.scratch_bytes >= 4 * M * K, (M, N, K, cus)
-                assert M > 128 or not r.gemm_few_rows, (M, N, K, cus)
+                assert R.GEMM_KERNELS[r.gemm_kernel] != "few_rows", (M, N, K, cus)
 
 
 def test_few_rows_past_one_round_of_a_small_device():

@@ -96,7 +96,7 @@ class CLinearRoute(ctypes.Structure):
     _fields_ = [
         ("kernel", c_uint32),
         ("splits", c_uint32),
-        ("gemm_few_rows", c_uint32),
+        ("gemm_kernel", c_uint32),
         ("reserved", c_uint32),
         ("scratch_bytes", c_uint64),
     ]

@@ -338,14 +338,16 @@ struct GemmArgs {
 uint32_t gemm_splits(int mode, const GemmArgs& g);
 uint32_t gemm_cus();  // CUs of the device
 size_t gemm_part_elems();
-// What a dense Plain launch that is given `part` runs on a device of `cus` CUs:
-// the few-row kernel or tiles, and its K splits.
+// Which kernel a launch runs (the 128 x 256 tile, the 256 x 256 one, the few-row
+// kernel, the 128 x 128 tile) and its K splits: gemm_plain_plan for a dense
+// Plain launch that is given `part` on a device of `cus` CUs.
 constexpr uint32_t kSlabMaxRows = 128;  // most rows of the few-row kernel
-struct PlainGemmPlan {
-    bool few_rows;
+enum class GemmKernel : uint32_t { Tile, Wide, Slab, Square };
+struct GemmPlan {
+    GemmKernel kernel;
     uint32_t splits;
 };
-PlainGemmPlan gemm_plain_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t cus);
+GemmPlan gemm_plain_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t cus);
 // The few-row kernel on f32 rows of A, which it splits itself (one segment of
 // W; a and W 16-byte aligned): `splits` as gemm_plain_plan gives them, `part`
 // needed where they are more than one. launch_slab_reduce adds up any Plain

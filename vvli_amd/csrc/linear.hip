@@ -437,8 +437,8 @@ LinearPlan linear_plan(uint32_t M, uint32_t N, uint32_t K, bool w_aligned, bool 
     if (linear_uses_gemv(M, N, K)) return p;
     const size_t sums = (size_t)M * N * sizeof(float);
     if (M <= kSlabMaxRows && w_aligned && x_aligned && !lean) {
-        const PlainGemmPlan g = gemm_plain_plan(M, N, K, cus);
-        if (g.few_rows && (M > kSkinnyMaxRows || slab_beats_skinny(M, N, K, g.splits, cus))) {
+        const GemmPlan g = gemm_plain_plan(M, N, K, cus);
+        if (g.kernel == GemmKernel::Slab && (M > kSkinnyMaxRows || slab_beats_skinny(M, N, K, g.splits, cus))) {
             p.kernel = LinearKernel::FewRows, p.splits = g.splits;
             p.payload = g.splits > 1 ? g.splits * sums : 0;
             return p;
@@ -654,7 +654,7 @@ int vvli_gpu_test_linear_route(uint32_t M, uint32_t N, uint32_t K, uint32_t cus,
     if (flags & VVLI_ROUTE_CAPTURED) p = captured_plan(p, linear_plan(M, N, K, aligned, true, true, cus));
     out->kernel = static_cast<uint32_t>(p.kernel);
     out->splits = p.splits;
-    out->gemm_few_rows = gemm_plain_plan(M, N, K, cus).few_rows;
+    out->gemm_kernel = static_cast<uint32_t>(gemm_plain_plan(M, N, K, cus).kernel);
     out->scratch_bytes = p.bytes();
     return VVLI_OK;
 }

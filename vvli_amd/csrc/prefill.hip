@@ -1335,13 +1335,6 @@ static hipError_t launch_gemm_wide(const GemmArgs& g, uint32_t cols, hipStream_t
     return vlaunch(gemm_wide_kernel<MODE>, grid, dim3(kGemmThreads), kWideLds, s, g);
 }
 
-// Which kernel a launch runs and its K splits.
-enum class GemmKernel { Tile, Wide, Slab, Square };
-struct GemmPlan {
-    GemmKernel kernel;
-    uint32_t splits;
-};
-
 // Splits of the few-row kernel: enough items for a block per CU, the fewest
 // splits with the same longest K range, at most kMaxPartSplits.
 static uint32_t slab_splits(uint32_t tiles, uint32_t K, uint32_t M, uint32_t cus) {
@@ -1379,12 +1372,11 @@ static GemmPlan gemm_plan(int mode, const GemmArgs& g, uint32_t cus) {
 
 uint32_t gemm_splits(int mode, const GemmArgs& g) { return gemm_plan(mode, g, gemm_cus()).splits; }
 
-PlainGemmPlan gemm_plain_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t cus) {
+GemmPlan gemm_plain_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t cus) {
     static float there;  // only that `part` is given counts
     GemmArgs g;
     g.M = M, g.N = N, g.K = K, g.ldo = N, g.part = &there;
-    const GemmPlan p = gemm_plan(kGemmPlain, g, cus);
-    return {p.kernel == GemmKernel::Slab, p.splits};
+    return gemm_plan(kGemmPlain, g, cus);
 }
 
 template <int MODE, int MT, int KC, int ST, int WM, int WN, bool F32A>

@@ -412,6 +412,7 @@ def linear(dW: int, dX: int, dY: int, M: int, N: int, K: int, dBias: int | None 
 
 
 LINEAR_KERNELS = ("gemv", "skinny", "few_rows", "tiles")
+GEMM_KERNELS = ("128x256", "256x256", "few_rows", "128x128")
 
 
 def linear_route(M: int, N: int, K: int, cus: int = 256, captured: bool = False, lean: bool = False,
