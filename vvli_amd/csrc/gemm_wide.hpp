@@ -6,14 +6,15 @@
 // MFMA tiles of 16 x 16) per CU, K steps of 32, no K split.
 //
 // Why this tile: at 128 x 256 a K step moves 96 KiB of fragments out of LDS
-// and 32 KiB into it for 1024 cycles of MFMA per SIMD, which is all that a
-// CU's LDS moves in that time (128 bytes a cycle). Here it is 128 + 48 KiB for
-// 2048 cycles, two thirds of it, and 27 % less copied per product. Two waves
+// and 32 KiB into it for 1024 cycles of MFMA per SIMD. Here it is 128 + 48 KiB
+// for 2048 cycles: two thirds of it, and 27 % less copied per product. Two waves
 // per SIMD stay (128 accumulators + 96 fragment registers + addresses: 251 of
 // 256), since one wave per SIMD hides too little of the LDS latency.
 // Measured (gate/up at 2048 rows of 2048 x 8192, split activations counted
 // twice): 264 -> 217 us, 1040 -> 1265 TFLOP/s on the matrix cores; a large
-// bf16 product of the library's reaches 1347 on the same card.
+// bf16 product of the library's reaches 1347 on the same card. Counters there:
+// matrix cores busy 59 % of the cycles (43 % on 128 x 256), no bank conflicts,
+// the clock at 2.1 GHz where lighter kernels run at 2.4.
 //
 // Stage (48 KiB): [A hi 16 KiB | A lo 16 KiB | W 16 KiB], rows of 64 bytes
 // swizzled as in the 128 x 256 tile; three stages (144 KiB). A wave holds all

@@ -1283,8 +1283,9 @@ size_t gemm_part_elems() { return gemm_part_elems(gemm_cus()); }
 // us and, per K step of 32, 0.90 on 128 x 256, 1.48 on 256 x 256, 0.47 on
 // 128 x 128; a K split adds its partial sums, written and read once by their
 // consumer (5 MB per us, and up to 3 us for a launch or its loads), or zeroing
-// and atomic adds (1.7 MB per us). Fitted to linear on each of the three (us, 128 x
-// 256 / 256 x 256 / 128 x 128): 2048 x 8192 x 2048 147 / 118 / 158, with K 512
+// and atomic adds (1.7 MB per us). Fitted to linear (its split pass included, all
+// on one box; others are up to 15 % off) on each of the three (us, 128 x 256 /
+// 256 x 256 / 128 x 128): 2048 x 8192 x 2048 147 / 118 / 158, with K 512
 // 60 / 47 / 70; 2048 x 4096 x 2048 80 / 100 / 87; 512 x 8192 x 2048 55 / 97 /
 // 46; 512 x 18000 x 1000 83 / 63 / 78; 200 x 2048 x 8192 50 / 320 / 35;
 // 130 x 1000 x 4000 29 / 159 / 26.
@@ -1348,7 +1349,8 @@ static GemmPlan gemm_plan(int mode, const GemmArgs& g, uint32_t cus) {
     const uint32_t cols = mode == kGemmGateUp ? 2 * g.N : g.N;
     // Few rows: the slab kernel. Up to 64 rows always (one layer of the 1B
     // shape at 45 rows: gate/up 36 -> 20 us with its zeroing and SwiGLU passes,
-    // o and down 17 -> 9.5, q|k|v 15 -> 9.5); from 65 to 128 while its items
+    // o and down 17 -> 9.5, q|k|v 15 -> 9.5; two Qwen2.5-7B layers, whose 592
+    // items of gate/up are three uneven rounds, 540 -> 414 us at 64 rows); from 65 to 128 while its items
     // are one round of at most 40 K chunks (linear at 65 / 128 rows, us, this
     // and the tiles with their split pass: 8192 x 2048 23.7 / 25.3 and 25.8 /
     // 29.2; 16384 x 2560, 40 chunks, 40.3 / 41.9 and 37.0 / 44.4; 4096 x 11008,
